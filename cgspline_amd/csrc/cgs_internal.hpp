@@ -130,7 +130,6 @@ constexpr int kPersistKernels = 7;
 struct PersistArgs
 {
     float2* stack;          // lanes × CGS_CLIP_STACK × 20 float2
-    uint32_t lanes;         // grid × 256
     unsigned int* counter;  // zeroed before the launch
     uint32_t grid;
 };
@@ -157,7 +156,7 @@ hipError_t launchTraceAny(const SceneDev& sc, const PersistArgs& pa, const cgs_r
 // the pair can be captured in a graph).
 // big: some job's scene has a wide-hashed BVH or a surface cull tree.
 hipError_t launchTraceBatch(const BatchJob* jobs, uint32_t njobs, uint32_t total, uint32_t chunk, float2* stack,
-                            uint32_t lanes, unsigned int* counter, uint32_t grid, unsigned long long* overflow, hipStream_t s,
+                            unsigned int* counter, uint32_t grid, unsigned long long* overflow, hipStream_t s,
                             const TraceMode& m, bool big);
 hipError_t launchClipBatch(const PersistArgs& pa, const cgs_ray* rays, const float* patches, uint32_t n, float tol,
                            cgs_hit* hits, hipStream_t s);
@@ -173,7 +172,7 @@ hipError_t launchPick(const SceneDev& sc, const PersistArgs& pa, const cgs_ray* 
 // `one` non-null every job is on that scene.  The counter must be zero at
 // launch.  counts (nullable): cgs_ray_counts, accumulated.
 hipError_t launchShade(const SceneDev* one, const ShadeJob* jobs, uint32_t njobs, uint32_t total, uint32_t chunk,
-                       float2* stack, uint32_t lanes, unsigned int* counter, uint32_t grid, unsigned long long* counts,
+                       float2* stack, unsigned int* counter, uint32_t grid, unsigned long long* counts,
                        hipStream_t s);
 // kRender reads its camera, options and output pointers from `argsDev`, a
 // device block of kRenderArgsBytes that launchRender fills on stream `s`.

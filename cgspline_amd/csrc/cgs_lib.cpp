@@ -146,7 +146,6 @@ static cgs_status persistArgs(cgs_ctx* ctx, PersistKernel k, hipStream_t s, uint
         ctx->stackLanes = lanes;
     }
     pa.stack = ctx->dStack;
-    pa.lanes = (uint32_t)lanes;
     pa.counter = ctx->dCounters + ki;
     pa.grid = ctx->grid[ki];
     if (ctx->persistLaunched) HIP_TRY(hipStreamWaitEvent(s, ctx->persistDone, 0));
@@ -1494,7 +1493,7 @@ cgs_status cgs_shade(cgs_ctx* ctx, cgs_scene* sc, const cgs_ray* rays, uint32_t 
     // so it has been read when the call returns; the copy itself runs in
     // stream order after the previous persistent launch.
     HIP_TRY(hipMemcpyAsync(ctx->dShadeJob, &job, sizeof job, hipMemcpyHostToDevice, s));
-    HIP_TRY(launchShade(&view, ctx->dShadeJob, 1, n, 64, pa.stack, pa.lanes, pa.counter, pa.grid,
+    HIP_TRY(launchShade(&view, ctx->dShadeJob, 1, n, 64, pa.stack, pa.counter, pa.grid,
                         (unsigned long long*)counts, s));
     return persistEnd(ctx, s);
 }
@@ -1608,8 +1607,7 @@ static cgs_status traceBatch(cgs_ctx* ctx, const cgs_batch_job* jobs, uint32_t n
     if ((st = persistArgs(ctx, PersistKernel::Batch, s, total, pa)) != CGS_OK) return st;
     HIP_TRY(hipMemcpyAsync(ctx->batchTable.p, table.data(), table.size() * sizeof(BatchJob), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s)); // the host table is released on return
-    HIP_TRY(launchTraceBatch(ctx->batchTable.as<BatchJob>(), (uint32_t)table.size(), total, chunk, pa.stack,
-                             std::min<uint32_t>(pa.lanes, (uint32_t)ctx->stackLanes), pa.counter, grid,
+    HIP_TRY(launchTraceBatch(ctx->batchTable.as<BatchJob>(), (uint32_t)table.size(), total, chunk, pa.stack, pa.counter, grid,
                              ctx->dOverflow, s, mode, anyBig(table)));
     HIP_TRY(hipEventRecord(ctx->batchDone, s));
     ctx->batchLaunched = true;
@@ -1667,7 +1665,7 @@ cgs_status cgs_batch_create(cgs_ctx* ctx, const cgs_batch_job* jobs, uint32_t nj
     if (e == hipSuccess) e = launchFill(b->counter.as<uint32_t>(), 0u, 1, cs);
     if (e == hipSuccess)
         e = launchTraceBatch(b->table.as<BatchJob>(), (uint32_t)table.size(), total, ctx->batchChunk,
-                             b->stack.as<float2>(), lanes, b->counter.as<unsigned int>(), grid,
+                             b->stack.as<float2>(), b->counter.as<unsigned int>(), grid,
                              b->overflow.as<unsigned long long>(), cs, ctx->batchMode, anyBig(table));
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(cs, &g);
@@ -2234,7 +2232,7 @@ struct cgs_server
             bool big = false;
             for (size_t k = 0; k < nTrace; k++) big |= jt[k].sc.big != 0;
             if ((e = launchTraceBatch(sl.table.as<BatchJob>(), (uint32_t)nTrace, traceRays, chunk, sl.stack.as<float2>(),
-                                      lanes, sl.counter.as<unsigned int>(), grid, sl.overflow.as<unsigned long long>(),
+                                      sl.counter.as<unsigned int>(), grid, sl.overflow.as<unsigned long long>(),
                                       sl.stream, TraceMode {}, big)) != hipSuccess)
                 return e;
         }
@@ -2244,7 +2242,7 @@ struct cgs_server
                                     sl.stream)) != hipSuccess)
                 return e;
             if ((e = launchShade(nullptr, sl.shadeTable.as<ShadeJob>(), (uint32_t)nShade, shadeRays, chunk,
-                                 sl.stack.as<float2>(), lanes, sl.counter.as<unsigned int>() + 1, shadeGrid, nullptr,
+                                 sl.stack.as<float2>(), sl.counter.as<unsigned int>() + 1, shadeGrid, nullptr,
                                  sl.stream)) != hipSuccess)
                 return e;
         }

@@ -18,7 +18,8 @@
 namespace cgs
 {
 
-constexpr float kClipTol = 0x1p-12f; // Spline.h:493
+constexpr float kClipTol = 0x1p-12f;  // Spline.h:493
+constexpr float kClipTol2 = 0x1p-24f; // tolSquare(kClipTol)
 
 // Leaf method of the ray queries.  Clip: Bézier clipping (the reference's
 // leaf call, Primitive.cu:234,260); ClipCapped: the same stopped after a
@@ -34,7 +35,7 @@ enum LeafMethod : int
 
 struct TraceParams
 {
-    float tol;          // clipping tolerance (Spline.h:493 default 2^-12)
+    float tol2;         // tolSquare of the clipping tolerance (Spline.h:493 default 2^-12)
     float threshold;    // subdivision threshold (Spline.h:500 default 2^-4)
     uint32_t maxIters;  // ClipCapped: loop passes per patch test
 };
@@ -234,9 +235,9 @@ CGS_DEV bool leafTest(const float4* __restrict__ S, const ClipRay& cr, const Tra
     if constexpr (METHOD == Subdiv)
         f = subdividePatch<ANY>(S, cr.o, cr.d, tp.threshold, best, bu, bv, overflow);
     else if constexpr (METHOD == ClipCapped)
-        f = clipPatch<ANY, true>(S, cr, tp.tol, best, bu, bv, stk, overflow, tp.maxIters);
+        f = clipPatch<ANY, true>(S, cr, tp.tol2, best, bu, bv, stk, overflow, tp.maxIters);
     else
-        f = clipPatch<ANY>(S, cr, tp.tol, best, bu, bv, stk, overflow);
+        f = clipPatch<ANY>(S, cr, tp.tol2, best, bu, bv, stk, overflow);
     return f;
 }
 
@@ -365,7 +366,7 @@ CGS_DEV bool surfaceClosestCulled(const SceneDev& sc, const DevBVH& surf, const 
         float t = lr.max, u = 0.0f, v = 0.0f;
         bool f;
         if constexpr (METHOD == Clip)
-            f = clipPatch<false>(S, cr, kClipTol, t, u, v, stk, overflow);
+            f = clipPatch<false>(S, cr, kClipTol2, t, u, v, stk, overflow);
         else
             f = leafTest<METHOD, false>(S, cr, tp, t, u, v, stk, overflow);
         if (overflow) return false;
@@ -435,7 +436,7 @@ CGS_DEV bool surfaceAnyCulled(const SceneDev& sc, const DevBVH& surf, const Loca
         float best = lr.max, bu, bv;
         bool f;
         if constexpr (METHOD == Clip)
-            f = clipPatch<true>(S, cr, kClipTol, best, bu, bv, stk, overflow);
+            f = clipPatch<true>(S, cr, kClipTol2, best, bu, bv, stk, overflow);
         else
             f = leafTest<METHOD, true>(S, cr, tp, best, bu, bv, stk, overflow);
         if (overflow) return false;
@@ -484,7 +485,7 @@ CGS_DEV bool objectClosest(const SceneDev& sc, const Rings& rg, uint32_t i, V3 o
         // the default keeps the direct call: routing it through leafTest
         // costs the render and trace kernels hundreds of spilled VGPRs
         if constexpr (METHOD == Clip)
-            f = clipPatch<false>(S, cr, kClipTol, lt, lu, lv, stk, overflow);
+            f = clipPatch<false>(S, cr, kClipTol2, lt, lu, lv, stk, overflow);
         else
             f = leafTest<METHOD, false>(S, cr, tp, lt, lu, lv, stk, overflow);
         if (f) lp = pid;
@@ -526,7 +527,7 @@ CGS_DEV bool objectAny(const SceneDev& sc, const Rings& rg, uint32_t i, V3 o, V3
         const float4* S = sc.patches + 16 * (size_t)(surf.patchBase + pid);
         float best = lr.max, bu, bv;
         if constexpr (METHOD == Clip)
-            return clipPatch<true>(S, cr, kClipTol, best, bu, bv, stk, overflow);
+            return clipPatch<true>(S, cr, kClipTol2, best, bu, bv, stk, overflow);
         else
             return leafTest<METHOD, true>(S, cr, tp, best, bu, bv, stk, overflow);
     }, NodeCache {nullptr, 0}, rg.bot);
@@ -608,7 +609,7 @@ CGS_DEV bool anyCulled(const SceneDev& sc, const Rings& rg, V3 o, V3 d, V3 Dinv,
 // could depend on the visit order) by the reference's top-level traversal.
 template<int METHOD = Clip, bool BIG = true>
 CGS_DEV ClosestHit sceneClosest(const SceneDev& sc, const NodeCache& nc, const Rings& rg, V3 o, V3 d, float tmax,
-                                const ClipStack& stk, bool& overflow, const TraceParams& tp = {kClipTol, 0x1p-4f, 0})
+                                const ClipStack& stk, bool& overflow, const TraceParams& tp = {kClipTol2, 0x1p-4f, 0})
 {
     if (sc.top.cullRoot != EMPTY)
     {
@@ -640,7 +641,7 @@ CGS_DEV ClosestHit sceneClosest(const SceneDev& sc, const NodeCache& nc, const R
 // origin->seen tells whether the traversal reached it (OriginSkip).
 template<int METHOD = Clip, bool BIG = true>
 CGS_DEV bool sceneAny(const SceneDev& sc, const NodeCache& nc, const Rings& rg, V3 o, V3 d, float tmax,
-                      const ClipStack& stk, bool& overflow, const TraceParams& tp = {kClipTol, 0x1p-4f, 0},
+                      const ClipStack& stk, bool& overflow, const TraceParams& tp = {kClipTol2, 0x1p-4f, 0},
                       OriginSkip* origin = nullptr)
 {
     if (sc.top.cullRoot != EMPTY)
@@ -671,7 +672,7 @@ CGS_DEV bool originAny(const SceneDev& sc, const OriginSkip& origin, V3 o, V3 d,
     const ClipRay cr = makeClipRay(lr.o, versor3(lr.d));
     const float4* S = sc.patches + 16 * (size_t)(surf.patchBase + origin.patch);
     float best = lr.max, bu, bv;
-    return clipPatch<true>(S, cr, kClipTol, best, bu, bv, stk, overflow);
+    return clipPatch<true>(S, cr, kClipTol2, best, bu, bv, stk, overflow);
 }
 
 // Device totals of the work events (CGS_WORK_COUNTS builds).  The sampled
@@ -730,7 +731,6 @@ CGS_DEV void addWave(unsigned long long* ctr, unsigned long long v)
 struct Persist
 {
     float2* stack;
-    uint32_t lanes;
     unsigned int* counter;
 };
 
@@ -758,7 +758,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
     const NodeCache nc = stageTopLevel(sc, topLds);
     const Rings rg = laneRings(ringLds);
     const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl, ps.lanes);
+    const ClipStack stk = clipStackFor(ps.stack, gl);
     unsigned long long nOverflow = 0;
     for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
     {
@@ -799,7 +799,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
     const NodeCache nc = stageTopLevel(sc, topLds);
     const Rings rg = laneRings(ringLds);
     const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl, ps.lanes);
+    const ClipStack stk = clipStackFor(ps.stack, gl);
     unsigned long long nOverflow = 0;
     for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
     {
@@ -827,7 +827,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
     unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
     const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl, ps.lanes);
+    const ClipStack stk = clipStackFor(ps.stack, gl);
     const NodeCache none {nullptr, 0};
     __shared__ uint32_t ringLds[kRingWords];
     const Rings rg = laneRings(ringLds);
@@ -889,11 +889,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
 #if !CGS_SAMPLED_TU
 // Batched doBezierClipping: ray r against patch r (Spline_BezierClipping.cu:46-114).
 __global__ __launch_bounds__(256) void kClipBatch(Persist ps, const cgs_ray* __restrict__ rays,
-                                                  const float4* __restrict__ patches, uint32_t n, float tol,
+                                                  const float4* __restrict__ patches, uint32_t n, float tol2,
                                                   cgs_hit* __restrict__ hits)
 {
     const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl, ps.lanes);
+    const ClipStack stk = clipStackFor(ps.stack, gl);
     for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
     {
         const uint32_t r = base + (threadIdx.x & 63);
@@ -902,7 +902,7 @@ __global__ __launch_bounds__(256) void kClipBatch(Persist ps, const cgs_ray* __r
         bool overflow = false;
         const ClipRay cr = makeClipRay({ray.ox, ray.oy, ray.oz}, versor3({ray.dx, ray.dy, ray.dz}));
         float t = ray.tmax, u = 0.0f, v = 0.0f;
-        bool f = clipPatch<false>(patches + 16 * (size_t)r, cr, tol, t, u, v, stk, overflow);
+        bool f = clipPatch<false>(patches + 16 * (size_t)r, cr, tol2, t, u, v, stk, overflow);
         hits[r] = {t, u, v, overflow ? CGS_PATCH_OVERFLOW : (f ? 1u : EMPTY)};
     }
 }
@@ -1087,7 +1087,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
     __shared__ uint32_t ringLds[kRingWords];
     const Rings rg = laneRings(ringLds);
     const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl, ps.lanes);
+    const ClipStack stk = clipStackFor(ps.stack, gl);
     const DevBVH surf = sc.surfaces[0];
     const BVHRef b = bvhRef(sc, surf);
     for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
@@ -1103,7 +1103,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
         {
             const bool f = hashIntersectAny<true>(b, o, d, ray.tmax, [&](uint32_t pid) -> bool {
                 float best = __builtin_inff(), bu, bv;
-                return clipPatch<true>(sc.patches + 16 * (size_t)(surf.patchBase + pid), cr, kClipTol, best, bu, bv, stk,
+                return clipPatch<true>(sc.patches + 16 * (size_t)(surf.patchBase + pid), cr, kClipTol2, best, bu, bv, stk,
                                        overflow);
             }, NodeCache {nullptr, 0}, rg.bot);
             occluded[r] = overflow ? 2u : (f ? 1u : 0u);
@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
             float t = ray.tmax, u = 0.0f, v = 0.0f;
             uint32_t patch = EMPTY;
             hashIntersect<true>(b, o, d, t, [&](uint32_t pid) -> bool {
-                const bool f = clipPatch<false>(sc.patches + 16 * (size_t)(surf.patchBase + pid), cr, kClipTol, t, u, v,
+                const bool f = clipPatch<false>(sc.patches + 16 * (size_t)(surf.patchBase + pid), cr, kClipTol2, t, u, v,
                                                 stk, overflow);
                 if (f) patch = pid;
                 return f;
@@ -1307,7 +1307,7 @@ CGS_DEV V3 rayRadiance(const SceneDev& sc, const NodeCache& nc, const Rings& rg,
             // the hit's own patch last (OriginSkip): the answer is the same
             OriginSkip origin {h.object, h.patch, false};
             const V3 so = add3(Pt, mul3(*eps, L));
-            if (sceneAny<Clip, BIG>(sc, nc, rg, so, L, d, stk, overflow, {kClipTol, 0x1p-4f, 0}, &origin)) continue;
+            if (sceneAny<Clip, BIG>(sc, nc, rg, so, L, d, stk, overflow, {kClipTol2, 0x1p-4f, 0}, &origin)) continue;
             if (origin.seen && originAny(sc, origin, so, L, d, stk, overflow)) continue;
             V3 H = versor3(add3(L, V));
             float dotHN = dot3(H, N);
@@ -1383,7 +1383,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
     const NodeCache nc = stageTopLevel(sc, topLds);
     const Rings rg = laneRings(ringLds);
     const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl, ps.lanes);
+    const ClipStack stk = clipStackFor(ps.stack, gl);
     const uint32_t lane = threadIdx.x & 63;
     uint32_t nItems;
     {
@@ -1486,7 +1486,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
     }
     const Rings rg = laneRings(ringLds);
     const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl, ps.lanes);
+    const ClipStack stk = clipStackFor(ps.stack, gl);
     uint32_t nPrimary = 0, nShadow = 0, nSecondary = 0, nOverflow = 0;
     while (true)
     {
@@ -1552,7 +1552,7 @@ namespace cgs
 {
 hipError_t launchRenderSampled(const SceneDev& sc, const PersistArgs& pa, const void* argsDev, hipStream_t s)
 {
-    Persist ps {pa.stack, pa.lanes, pa.counter};
+    Persist ps {pa.stack, pa.counter};
     hipLaunchKernelGGL((kRender<true, true>), dim3(pa.grid), dim3(256), 0, s, sc, ps, (const RenderArgs*)argsDev);
     return hipGetLastError();
 }
@@ -1590,16 +1590,34 @@ hipError_t persistentGrid(PersistKernel k, uint32_t& blocksPerCU)
 // where the default kernels do not).  The default kernels clip at the fixed
 // 2^-12, so a clipping run with another tolerance takes the capped kernels
 // with a cap no run reaches (2^32 - 1 passes).
+// The least float x whose square root is at least tol, so that
+// sqrt(x) < tol is x < tolSquare(tol) (the correctly rounded square root is
+// monotone): two compares per clipping pass instead of two square roots.
+// 0 where no square root is below tol (tol <= 0 or NaN).
+static float tolSquare(float tol)
+{
+    if (!(tol > 0.0f)) return 0.0f;
+    const uint32_t inf = 0x7F800000u;
+    uint32_t lo = 0u, hi = inf;      // sqrt(lo) < tol; hi is inf or sqrt(hi) >= tol
+    while (hi - lo > 1u)
+    {
+        const uint32_t m = lo + (hi - lo) / 2u;
+        if (__builtin_sqrtf(std::bit_cast<float>(m)) < tol) lo = m;
+        else hi = m;
+    }
+    return std::bit_cast<float>(hi);
+}
+
 static TraceParams traceParams(const TraceMode& m)
 {
-    return {m.tol, m.threshold, m.maxIters ? m.maxIters : 0xFFFFFFFFu};
+    return {tolSquare(m.tol), m.threshold, m.maxIters ? m.maxIters : 0xFFFFFFFFu};
 }
 
 hipError_t launchTraceClosest(const SceneDev& sc, const PersistArgs& pa, const cgs_ray* rays, uint32_t n, cgs_hit* hits,
                               int32_t* objects, unsigned long long* overflow, hipStream_t s, const TraceMode& m)
 {
     if (n == 0) return hipSuccess;
-    Persist ps {pa.stack, pa.lanes, pa.counter};
+    Persist ps {pa.stack, pa.counter};
     const TraceParams tp = traceParams(m);
 #define CGS_LAUNCH_CLOSEST(M, P) \
     hipLaunchKernelGGL((kTraceClosest<M, P>), dim3(pa.grid), dim3(256), 0, s, sc, ps, rays, n, hits, objects, overflow, tp)
@@ -1623,7 +1641,7 @@ hipError_t launchTraceAny(const SceneDev& sc, const PersistArgs& pa, const cgs_r
                           unsigned long long* overflow, hipStream_t s, const TraceMode& m)
 {
     if (n == 0) return hipSuccess;
-    Persist ps {pa.stack, pa.lanes, pa.counter};
+    Persist ps {pa.stack, pa.counter};
     const TraceParams tp = traceParams(m);
     if (m.method == CGS_METHOD_SUBDIVISION)
         hipLaunchKernelGGL((kTraceAny<Subdiv>), dim3(pa.grid), dim3(256), 0, s, sc, ps, rays, n, occluded, overflow, tp);
@@ -1635,11 +1653,11 @@ hipError_t launchTraceAny(const SceneDev& sc, const PersistArgs& pa, const cgs_r
 }
 
 hipError_t launchTraceBatch(const BatchJob* jobs, uint32_t njobs, uint32_t total, uint32_t chunk, float2* stack,
-                            uint32_t lanes, unsigned int* counter, uint32_t grid, unsigned long long* overflow, hipStream_t s,
+                            unsigned int* counter, uint32_t grid, unsigned long long* overflow, hipStream_t s,
                             const TraceMode& m, bool big)
 {
     if (total == 0) return hipSuccess;
-    Persist ps {stack, lanes, counter};
+    Persist ps {stack, counter};
     const TraceParams tp = traceParams(m);
     // the default method has a kernel without the wide-hash and surface-cull paths
     if (!big && m.method != CGS_METHOD_SUBDIVISION && !m.maxIters && m.tol == kClipTol && !m.polish)
@@ -1670,8 +1688,8 @@ hipError_t launchClipBatch(const PersistArgs& pa, const cgs_ray* rays, const flo
                            cgs_hit* hits, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    Persist ps {pa.stack, pa.lanes, pa.counter};
-    hipLaunchKernelGGL(kClipBatch, dim3(pa.grid), dim3(256), 0, s, ps, rays, (const float4*)patches, n, tol, hits);
+    Persist ps {pa.stack, pa.counter};
+    hipLaunchKernelGGL(kClipBatch, dim3(pa.grid), dim3(256), 0, s, ps, rays, (const float4*)patches, n, tolSquare(tol), hits);
     return hipGetLastError();
 }
 
@@ -1701,11 +1719,11 @@ hipError_t launchSubpatch(const float* patches, const float* ranges, uint32_t n,
 }
 
 hipError_t launchShade(const SceneDev* one, const ShadeJob* jobs, uint32_t njobs, uint32_t total, uint32_t chunk,
-                       float2* stack, uint32_t lanes, unsigned int* counter, uint32_t grid, unsigned long long* counts,
+                       float2* stack, unsigned int* counter, uint32_t grid, unsigned long long* counts,
                        hipStream_t s)
 {
     if (total == 0 || njobs == 0) return hipSuccess;
-    Persist ps {stack, lanes, counter};
+    Persist ps {stack, counter};
     if (one)
         hipLaunchKernelGGL(kShade<true>, dim3(grid), dim3(256), 0, s, *one, jobs, njobs, total, chunk, ps, counts);
     else
@@ -1718,7 +1736,7 @@ hipError_t launchPick(const SceneDev& sc, const PersistArgs& pa, const cgs_ray* 
                       uint32_t* occluded, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    Persist ps {pa.stack, pa.lanes, pa.counter};
+    Persist ps {pa.stack, pa.counter};
     if (occluded)
         hipLaunchKernelGGL(kPick<true>, dim3(pa.grid), dim3(256), 0, s, sc, ps, rays, n, hits, occluded);
     else
@@ -1748,7 +1766,7 @@ hipError_t launchRender(const SceneDev& sc, const PersistArgs& pa, const float* 
     // so it has been read when the call returns.
     hipError_t e = hipMemcpyAsync(argsDev, &ra, sizeof ra, hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return e;
-    Persist ps {pa.stack, pa.lanes, pa.counter};
+    Persist ps {pa.stack, pa.counter};
     if (samples > 0) return launchRenderSampled(sc, pa, argsDev, s);
     if (sc.big)
         hipLaunchKernelGGL(kRender<true>, dim3(pa.grid), dim3(256), 0, s, sc, ps, (const RenderArgs*)argsDev);
