@@ -341,256 +341,6 @@ CGS_DEV ClipStack clipStackFor(float2* buf, uint32_t lane)
     return {buf + (size_t)(lane >> 6) * (CGS_CLIP_STACK * kStackWords * 64) + (lane & 63)};
 }
 
-// doBezierClipping with host semantics (Spline_BezierClipping.cu:46-114,
-// 174-445).  S: the 16 control points (global).  best/bu/bv: current hit,
-// updated by accepted candidates (t < best && V·d > 0).  With ANY the test
-// stops at the first accepted candidate (the caller only needs "found").
-// tol2 is the clipping tolerance's tolSquare: a region's size is compared
-// squared.
-// Returns found; sets overflow when the region stack is exhausted.
-// What bounds it is the instruction count of a pass, on the one lane that a
-// wave's slowest patch test keeps busy as on full waves.  Convergence by
-// squared sizes (no square roots), maxNum/minNum envelopes, straight-line
-// hull edges, one de Casteljau step for a split's two halves and stack words
-// at constant offsets took 200,000 (ray, patch) pairs from 752 to 571 us, the
-// 1M-patch frame from 14.0 to 10.8 ms and a 64-ray pick from 111 to 97 us.
-// CAPPED (an opt-in mode with no counterpart in the reference): the test
-// stops after maxIters passes of its loop and keeps what it found so far.
-template<bool ANY, bool CAPPED = false>
-CGS_DEV bool clipPatch(const float4* __restrict__ S, const ClipRay& R, float tol2, float& best, float& bu, float& bv,
-                       const ClipStack& stk, bool& overflow, uint32_t maxIters = 0)
-{
-    CGS_COUNT(kWorkPatch);
-    V2 p[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-    {
-        float4 q = S[i];
-        V3 D {q.x - R.o.x, q.y - R.o.y, q.z - R.o.z};
-        p[i] = {dot3(R.ax0, D), dot3(R.ax1, D)};
-    }
-    // 0 * x is NaN for the infinities and NaN
-    float fin = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; i++) fin += 0.0f * p[i].x + 0.0f * p[i].y;
-    const bool finite = fin == 0.0f;
-    V2 mn {0.0f, 0.0f}, mx {1.0f, 1.0f}, sz {1.0f, 1.0f};
-    bool vside = false;
-    int sp = 0; // entries stored below the current one
-    bool found = false;
-
-    auto onHit = [&](float eu, float ev) -> bool
-    {
-        CGS_COUNT(kWorkOnHit);
-        float4 X = interpolateMat(S, eu, ev);
-        V3 V = sub3(project4(X), R.o);
-        float t = len3(V);
-        if (t < best && dot3(V, R.d) > 0.0f)
-        {
-            best = t;
-            bu = eu;
-            bv = ev;
-            return true;
-        }
-        return false;
-    };
-
-    // The working patch is kept in the orientation of the current cut side:
-    // natural (p[4j+i] = point(i,j)) while clipping in u, transposed while
-    // clipping in v, so the curves being cut are always the rows p[4r..4r+3]
-    // and one code path serves both sides.  Transposing moves values only;
-    // every formula below gives the natural-orientation result bit for bit:
-    // the tolerance diagonals p3-p12 and p15-p0 change at most by an exact
-    // negation, L = (p15-p0) + (p12-p3) in transposed storage equals
-    // (p15-p0) - (p12-p3) in natural storage (x + (-y) == x - y), and the
-    // envelope visits the same points in the same order.
-    uint32_t iters = 0;
-    while (true)
-    {
-        if (CAPPED && iters++ >= maxIters) break;
-        bool pop = false;
-        V2 t0 {p[3].x - p[12].x, p[3].y - p[12].y};
-        V2 t1 {p[15].x - p[0].x, p[15].y - p[0].y};
-        if (t0.x * t0.x + t0.y * t0.y < tol2 && t1.x * t1.x + t1.y * t1.y < tol2)
-        {
-            CGS_COUNT(kWorkConverged);
-            // approximateIntersection (Spline.h:739-765) on the natural corners
-            const V2 c30 = vside ? p[12] : p[3], c03 = vside ? p[3] : p[12];
-            V2 c;
-            if (triangleOrigin(c, p[0], c30, c03))
-                found |= onHit(mn.x + c.x * sz.x, mn.y + c.y * sz.y);
-            if (triangleOrigin(c, p[15], c03, c30))
-                found |= onHit(mx.x - c.x * sz.x, mx.y - c.y * sz.y);
-            if (ANY && found) break;
-            pop = true;
-        }
-        else
-        {
-            V2 L {p[15].x - p[0].x, p[15].y - p[0].y};
-            const V2 Dv {p[12].x - p[3].x, p[12].y - p[3].y};
-            L = {L.x + Dv.x, L.y + Dv.y};
-            L = normalize2(L);
-            const V2 N {-L.y, L.x};
-            // signed distances N·p folded into the envelope as they are computed
-            float ytop[4], ybot[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-            {
-                const float d0 = N.x * p[i].x + N.y * p[i].y;
-                ybot[i] = d0;
-                ytop[i] = d0;
-#pragma unroll
-                for (int k = 1; k < 4; k++)
-                {
-                    const float dk = N.x * p[4 * k + i].x + N.y * p[4 * k + i].y;
-                    // maxNum / minNum: as fmax_ / fmin_ but for the sign of a
-                    // zero, which the hull below does not depend on (it enters
-                    // differences, compares, and quotients times an abscissa
-                    // that is added to a value never -0)
-                    ytop[i] = __builtin_fmaxf(ytop[i], dk);
-                    ybot[i] = __builtin_fminf(ybot[i], dk);
-                }
-            }
-            float lower = 1.0f, upper = 0.0f;
-            const float o1 = 1.0f / 3.0f, o2 = 2.0f / 3.0f;
-            const V2 hull[7] {{o2, ybot[2]}, {1.0f, ybot[3]}, {1.0f, ytop[3]}, {o2, ytop[2]},
-                              {o1, ytop[1]}, {0.0f, ytop[0]}, {0.0f, ybot[0]}};
-            V2 P1 {0.0f, ybot[0]};
-            V2 P2 {o1, ybot[1]};
-#pragma unroll
-            for (int h = 0; h < 7; h++)
-            {
-                const V2 P3 = hull[h];
-                const bool ccw = isCCW({P2.x - P1.x, P2.y - P1.y}, {P3.x - P1.x, P3.y - P1.y}) >= 0.0f;
-                hullEdge(lower, upper, P1, P2, ccw);
-                P1.x = ccw ? P2.x : P1.x;
-                P1.y = ccw ? P2.y : P1.y;
-                P2 = P3;
-            }
-            hullEdge(lower, upper, P1, P2, true);
-            lower = lower * 0x0FFp-8f;
-            upper = upper + (1.0f - upper) * 0x001p-8f;
-            const float delta = upper - lower;
-            if (delta < 0.0f)
-            {
-                CGS_COUNT(kWorkPrune);
-                pop = true;
-            }
-            else
-            {
-                // delta > 0.8: split in half, keep the upper half and push the
-                // lower half (Spline_BezierClipping.cu:373-409); otherwise clip
-                // to [lower, upper] (:410-432).  Both keep a slice of the rows.
-                const bool split = delta > 0.8f;
-                CGS_COUNT(split ? kWorkSplit : kWorkClip);
-                if (split && sp >= CGS_CLIP_STACK)
-                {
-                    overflow = true;
-                    break;
-                }
-                // region along the cut side (u: x, v: y)
-                const float smn = vside ? mn.y : mn.x, smx = vside ? mx.y : mx.x, ssz = vside ? sz.y : sz.x;
-                float nmn, nmx, nsz;
-                if (split)
-                {
-                    // the lower half, pushed for later: rows sliced to [0, 1/2],
-                    // stored transposed (the popped entry cuts the other side:
-                    // stored word 4c + r holds row r, point c); the upper half
-                    // stays.  One de Casteljau step at 1/2 gives both: the
-                    // reference slices the lower half first at 0 and the upper
-                    // last at 1, which multiply by 0 and 1 and change nothing
-                    // but the sign of a zero (no result depends on one) while
-                    // the points are finite; a net with an infinity or NaN
-                    // takes the two general slices.
-                    float2* e = stk.entry(sp);
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                    {
-                        V2 c0 = p[4 * r], c1 = p[4 * r + 1], c2 = p[4 * r + 2], c3 = p[4 * r + 3];
-                        if (finite)
-                        {
-                            halve1(c0.x, c1.x, c2.x, c3.x, p[4 * r].x, p[4 * r + 1].x, p[4 * r + 2].x);
-                            halve1(c0.y, c1.y, c2.y, c3.y, p[4 * r].y, p[4 * r + 1].y, p[4 * r + 2].y);
-                        }
-                        else
-                        {
-                            slice1(c0.x, c1.x, c2.x, c3.x, 0.0f, 1.0f, 0.5f, 0.5f);
-                            slice1(c0.y, c1.y, c2.y, c3.y, 0.0f, 1.0f, 0.5f, 0.5f);
-                            slice1(p[4 * r].x, p[4 * r + 1].x, p[4 * r + 2].x, p[4 * r + 3].x, 0.5f, 0.5f, 1.0f, 0.0f);
-                            slice1(p[4 * r].y, p[4 * r + 1].y, p[4 * r + 2].y, p[4 * r + 3].y, 0.5f, 0.5f, 1.0f, 0.0f);
-                        }
-                        e[64 * r] = make_float2(c0.x, c0.y);
-                        e[64 * (4 + r)] = make_float2(c1.x, c1.y);
-                        e[64 * (8 + r)] = make_float2(c2.x, c2.y);
-                        e[64 * (12 + r)] = make_float2(c3.x, c3.y);
-                    }
-                    const float hs = 0.5f * ssz;
-                    const float hm = smn + hs;
-                    const V2 emx = vside ? V2 {mx.x, hm} : V2 {hm, mx.y};
-                    const V2 psz = vside ? V2 {sz.x, hs} : V2 {hs, sz.y};
-                    e[64 * 16] = make_float2(mn.x, mn.y);
-                    e[64 * 17] = make_float2(emx.x, emx.y);
-                    e[64 * 18] = make_float2(psz.x, psz.y);
-                    e[64 * 19] = make_float2(vside ? 0.0f : 1.0f, 0.0f);
-                    sp++;
-                    nmn = hm;
-                    nmx = smx;
-                    nsz = hs;
-                }
-                else
-                {
-                    nmn = smn + ssz * lower;
-                    nmx = smx - ssz * (1.0f - upper);
-                    nsz = nmx - nmn;
-                    subpatchU2(p, lower, upper);
-                }
-                if (vside)
-                {
-                    mn.y = nmn;
-                    mx.y = nmx;
-                    sz.y = nsz;
-                }
-                else
-                {
-                    mn.x = nmn;
-                    mx.x = nmx;
-                    sz.x = nsz;
-                }
-                // the other side is cut next: transpose
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-#pragma unroll
-                    for (int c = r + 1; c < 4; c++)
-                    {
-                        const V2 t = p[4 * r + c];
-                        p[4 * r + c] = p[4 * c + r];
-                        p[4 * c + r] = t;
-                    }
-                vside = !vside;
-                continue;
-            }
-        }
-        if (pop)
-        {
-            if (sp == 0) break;
-            sp--;
-            const float2* e = stk.entry(sp);
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-            {
-                float2 q = e[64 * i];
-                p[i] = {q.x, q.y};
-            }
-            float2 r0 = e[64 * 16], r1 = e[64 * 17], r2 = e[64 * 18], r3 = e[64 * 19];
-            mn = {r0.x, r0.y};
-            mx = {r1.x, r1.y};
-            sz = {r2.x, r2.y};
-            vside = r3.x != 0.0f;
-        }
-    }
-    return found;
-}
-
 // Newton polish of a closest hit (an opt-in refinement with no counterpart
 // in the reference).  The clipper stops when the projected sub-patch is
 // below an absolute 2^-12, which leaves (u, v) uncertain by about
@@ -699,14 +449,6 @@ CGS_DEV bool polishHit64(const float4* __restrict__ S, const float4 (&w2l)[4], V
     u = (float)pu;
     v = (float)pv;
     return true;
-}
-
-// The same with the mode chosen per lane at run time.
-CGS_DEV bool clipPatchRT(const bool any, const float4* __restrict__ S, const ClipRay& R, float tol2, float& best,
-                         float& bu, float& bv, const ClipStack& stk, bool& overflow)
-{
-    return any ? clipPatch<true>(S, R, tol2, best, bu, bv, stk, overflow)
-               : clipPatch<false>(S, R, tol2, best, bu, bv, stk, overflow);
 }
 
 // ---------------------------------------------------------------------------
@@ -902,6 +644,18 @@ CGS_DEV uint32_t hashKey(const BVHRef& b, uint32_t key)
 // siblings are still postponed looks the key up in the perfect hash as
 // before.  The visited nodes and their order are unchanged.
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
+CGS_DEV uint32_t ldsOr(lds_u32* p, uint32_t v)
+{
+    return __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+CGS_DEV uint32_t ldsAdd(lds_u32* p, uint32_t v)
+{
+    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+CGS_DEV uint32_t ldsMin(lds_u32* p, uint32_t v)
+{
+    return __hip_atomic_fetch_min(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
 constexpr uint32_t kRingStride = 256;   // threads per workgroup: slot k of a lane is base[k * 256]
 
 struct SiblingRing
@@ -1028,60 +782,6 @@ CGS_DEV uint32_t nextLeafOct(int oct, const BVHRef& b, const NodeCache& nc, cons
     case 7: return nextLeaf<7, LOW, BIG>(b, nc, ring, o, Dinv, limit, st);
     default: return nextLeaf<-1, LOW, BIG>(b, nc, ring, o, Dinv, limit, st);
     }
-}
-
-// Stackless closest-hit traversal (rt/BVH.h:178-266).  `limit` is the
-// caller's hit.t (read through a reference so leaf hits tighten the culling);
-// `leaf(index)` tests one element and returns whether it improved the hit.
-// OCTANTS: specialise the node loop on the wave's direction octant (worth its
-// code size where a wave's rays are coherent: the top level, in world space).
-// LOW: the BVH's nodes lie in the first 4 GiB of the node array (loadNodeLow).
-template<bool OCTANTS = false, bool LOW = false, bool BIG = true, class Leaf>
-CGS_DEV bool hashIntersect(const BVHRef& b, V3 o, V3 dir, const float& limit, Leaf&& leaf,
-                           const NodeCache& nc = NodeCache {nullptr, 0}, const SiblingRing& ring = {nullptr, 0})
-{
-    const V3 Dinv {1.0f / dir.x, 1.0f / dir.y, 1.0f / dir.z};
-    TravState st {b.root, 1u, 0u, RingState {}};
-    const int oct = OCTANTS ? waveOctant(o, Dinv, b.finiteBoxes) : -1;
-    bool result = false;
-    uint32_t i;
-    while ((i = (OCTANTS ? nextLeafOct<LOW, BIG>(oct, b, nc, ring, o, Dinv, limit, st)
-                         : nextLeaf<-1, LOW, BIG>(b, nc, ring, o, Dinv, limit, st))) != EMPTY)
-    {
-        uint32_t e;
-        while ((e = b.indices[i]) != EMPTY)
-        {
-            CGS_COUNT(kWorkLeaf);
-            result |= leaf(e);
-            i++;
-        }
-        if (!ascend<BIG>(b, nc, ring, st)) break;
-    }
-    return result;
-}
-
-// Stackless any-hit traversal against `tmax` (rt/BVH.h:268-350).
-template<bool OCTANTS = false, bool LOW = false, bool BIG = true, class Leaf>
-CGS_DEV bool hashIntersectAny(const BVHRef& b, V3 o, V3 dir, float tmax, Leaf&& leaf,
-                              const NodeCache& nc = NodeCache {nullptr, 0}, const SiblingRing& ring = {nullptr, 0})
-{
-    const V3 Dinv {1.0f / dir.x, 1.0f / dir.y, 1.0f / dir.z};
-    TravState st {b.root, 1u, 0u, RingState {}};
-    const int oct = OCTANTS ? waveOctant(o, Dinv, b.finiteBoxes) : -1;
-    uint32_t i;
-    while ((i = (OCTANTS ? nextLeafOct<LOW, BIG>(oct, b, nc, ring, o, Dinv, tmax, st)
-                         : nextLeaf<-1, LOW, BIG>(b, nc, ring, o, Dinv, tmax, st))) != EMPTY)
-    {
-        uint32_t e;
-        while ((e = b.indices[i]) != EMPTY)
-        {
-            CGS_COUNT(kWorkLeaf);
-            if (leaf(e)) return true;
-            i++;
-        }
-        if (!ascend<BIG>(b, nc, ring, st)) break;
-    }
-    return false;
 }
 
 } // namespace cgs

@@ -13,6 +13,7 @@
 
 #include "cgs_internal.hpp"
 #include "cgs_scene_dev.hpp"
+#include "cgs_clip_wave.hpp"
 #include "cgs_sample.hpp"
 
 namespace cgs
@@ -226,20 +227,172 @@ CGS_DEV bool subdividePatch(const float4* __restrict__ S, V3 o, V3 d, float thre
     return found;
 }
 
-// One patch test of a scene query by the chosen leaf method.
-template<int METHOD, bool ANY>
-CGS_DEV bool leafTest(const float4* __restrict__ S, const ClipRay& cr, const TraceParams& tp, float& best, float& bu,
-                      float& bv, const ClipStack& stk, bool& overflow)
+// ---------------------------------------------------------------------------
+// Cull-tree enumeration (cgs_cull.cpp): the elements (objects or patches)
+// whose reference leaf box a ray passes, in the tree's near-to-far order
+// ---------------------------------------------------------------------------
+
+CGS_DEV bool cullable(V3 o, V3 Dinv)
 {
-    bool f;
-    if constexpr (METHOD == Subdiv)
-        f = subdividePatch<ANY>(S, cr.o, cr.d, tp.threshold, best, bu, bv, overflow);
-    else if constexpr (METHOD == ClipCapped)
-        f = clipPatch<ANY, true>(S, cr, tp.tol2, best, bu, bv, stk, overflow, tp.maxIters);
-    else
-        f = clipPatch<ANY>(S, cr, tp.tol2, best, bu, bv, stk, overflow);
-    return f;
+    auto ok = [](float oi, float di) { return __builtin_isfinite(oi) && __builtin_isfinite(di) && di != 0.0f; };
+    return ok(o.x, Dinv.x) && ok(o.y, Dinv.y) && ok(o.z, Dinv.z);
 }
+
+// A lane's place in one traversal, kept between two patch tests.  In a cull
+// tree: the next node (EMPTY: none) and the elements elem..elemEnd-1 of the
+// leaf being read.  In a hashed BVH: its TravState, and the next slot of the
+// leaf list being read (EMPTY: none).
+struct Walk
+{
+    TravState st;        // cull tree: st.node is the next node
+    uint32_t leaf;       // cull tree: elem
+    CGS_DEV uint32_t& elem() { return leaf; }
+    CGS_DEV uint32_t& elemEnd() { return st.key; }
+};
+CGS_DEV Walk cullWalk(uint32_t root) { return Walk {TravState {root, 0u, 0u, RingState {}}, 0u}; }
+CGS_DEV Walk hashWalk(uint32_t root) { return Walk {TravState {root, 1u, 0u, RingState {}}, EMPTY}; }
+
+// The next element whose reference leaf box the ray passes with entry
+// below tmax and at most lim; its entry in L0.  EMPTY at the end.
+CGS_DEV uint32_t cullNext(const SceneDev& sc, int oct, V3 o, V3 Dinv, float lim, float tmax, Walk& it, float& L0)
+{
+    uint32_t node = it.st.node, elem = it.elem(), elemEnd = it.elemEnd(), found = EMPTY;
+    while (true)
+    {
+        if (elem < elemEnd)
+        {
+            CGS_COUNT(kWorkCullElem);
+            const float4 a = sc.cullElems[2 * (size_t)elem], b = sc.cullElems[2 * (size_t)elem + 1];
+            elem++;
+            float l;
+            if (nodeIntersect<-1>(l, {a.x, a.y, a.z}, {b.x, b.y, b.z}, o, Dinv) && l < tmax && l <= lim)
+            {
+                L0 = l;
+                found = __float_as_uint(a.w);
+                break;
+            }
+            continue;
+        }
+        if (node == EMPTY) break;
+        CGS_COUNT(kWorkCullNode);
+        const float4 a = sc.cullNodes[2 * (size_t)node], b = sc.cullNodes[2 * (size_t)node + 1];
+        const uint2 l = sc.cullLinks[8 * (size_t)node + oct];
+        float tn;
+        const bool pass = nodeIntersect<-1>(tn, {a.x, a.y, a.z}, {b.x, b.y, b.z}, o, Dinv) && tn <= lim;
+        const uint32_t count = __float_as_uint(b.w);
+        if (pass && count)
+        {
+            elem = __float_as_uint(a.w);
+            elemEnd = elem + count;
+        }
+        node = pass && !count ? l.x : l.y;
+    }
+    it.st.node = node;
+    it.elem() = elem;
+    it.elemEnd() = elemEnd;
+    return found;
+}
+
+// The next element of a hashed BVH's stackless traversal (rt/BVH.h:178-350)
+// against `limit`: the closest-hit traversal's is the caller's nearest hit so
+// far, the any-hit one's the ray's end.  EMPTY at the end.  OCTANTS:
+// specialise the node loop on the wave's direction octant (worth its code
+// size where a wave's rays are coherent: in world space).  LOW: the BVH's
+// nodes lie in the first 4 GiB of the node array (loadNodeLow).
+template<bool OCTANTS, bool LOW, bool BIG>
+CGS_DEV uint32_t hashNext(const BVHRef& b, V3 o, V3 Dinv, float limit, const NodeCache& nc, const SiblingRing& ring,
+                          Walk& it)
+{
+    const int oct = OCTANTS ? waveOctant(o, Dinv, b.finiteBoxes) : -1;
+    while (true)
+    {
+        if (it.leaf != EMPTY)
+        {
+            const uint32_t e = b.indices[it.leaf];
+            if (e != EMPTY)
+            {
+                CGS_COUNT(kWorkLeaf);
+                it.leaf++;
+                return e;
+            }
+            it.leaf = EMPTY;
+            if (!ascend<BIG>(b, nc, ring, it.st)) return EMPTY;
+        }
+        it.leaf = OCTANTS ? nextLeafOct<LOW, BIG>(oct, b, nc, ring, o, Dinv, limit, it.st)
+                          : nextLeaf<-1, LOW, BIG>(b, nc, ring, o, Dinv, limit, it.st);
+        if (it.leaf == EMPTY) return EMPTY;
+    }
+}
+
+// How far beyond the nearest hit so far an object's box entry may lie and
+// the object still be tested: 2^-10 of the distance plus the origin's
+// magnitude, orders of magnitude above the FP32 rounding of a hit distance
+// or a box entry.
+CGS_DEV float cullLimit(float best, V3 o)
+{
+    const float mag = fmax_(__builtin_fabsf(o.x), fmax_(__builtin_fabsf(o.y), __builtin_fabsf(o.z)));
+    return best + (best + mag) * 0x1p-10f;
+}
+
+CGS_DEV int dirOctant(V3 Dinv)
+{
+    return (__builtin_signbit(Dinv.x) ? 1 : 0) | (__builtin_signbit(Dinv.y) ? 2 : 0) | (__builtin_signbit(Dinv.z) ? 4 : 0);
+}
+
+// A shadow ray's own surface patch, clipped last.  An any-hit answer is the
+// OR of the patch tests the traversal reaches, in whatever order, so a query
+// may pass over one patch, note that the traversal reached it (`seen`), and
+// clip it only if no other patch is hit (sceneQuery).  A shadow ray that
+// grazes its origin patch clips it for up to thousands of passes; one that
+// another patch occludes then never does.
+struct OriginSkip
+{
+    int32_t object;
+    uint32_t patch;
+    bool seen;
+};
+
+// ---------------------------------------------------------------------------
+// Scene queries (Context::intersect, RayTracer.cu:296-383)
+// ---------------------------------------------------------------------------
+//
+// One ray per lane, all lanes of a wave together: each lane walks the objects
+// its ray reaches and the patches of each (rt::intersect(BezierSurface),
+// Primitive.cu:222-268, on the object-local ray of RayTracer.cu:305-333) until
+// its next patch test, and then the wave clips all its lanes' patches in one
+// shared clip (clipWave), to which the lanes whose rays are done lend a hand.
+// With the test inside each lane's own traversal loops 11 of 64 lanes were
+// active on the 1M-patch frame, and a lane whose ray grazes a patch for
+// thousands of passes held its wave alone.
+//
+// Objects through the cull tree.  The reference's top-level traversal reaches
+// object X only if the ray passes X's leaf box with entry L0 below the hit
+// distance at that moment (rt/BVH.h:147-266), and every ancestor box contains
+// X's box, so it passes there whenever it passes X's (the slab test is
+// monotone in the box).  Each object's own result does not depend on the visit
+// order (its traversal starts from ray.max·|M d|, RayTracer.cu:311-314).  So:
+//  - any hit: the reference's answer is whether some object whose leaf box
+//    the ray passes with L0 < ray.max has a hit, in any order;
+//  - closest: enumerating every such object whose L0 is not far beyond the
+//    nearest hit found so far (a hit lies inside its object's box, up to
+//    rounding, for which the slack below leaves a wide margin) finds the
+//    nearest hit W.  The reference reaches W when L0_W < t_W (its limit is
+//    never below t_W), and then reports W unless another object has a hit at
+//    exactly t_W, where its visit order decides.
+// A lane starts its ray over by the reference's traversal for a tie, for
+// L0_W >= t_W, for a clip-stack overflow on the way (so that overflows are
+// reported as in the reference order), and takes it from the first for rays on
+// which the slab test could meet a NaN (a zero or non-finite direction
+// component, a non-finite origin) and scenes without the tree.
+//
+// The patches of a large surface through its own cull tree: the same argument
+// one level down.  A patch's clip accepts candidates by the running distance
+// only (t < best), so a patch's own nearest hit does not depend on the
+// distance its test starts from; every patch whose leaf box the local ray
+// passes near or before the nearest hit so far is clipped from the local ray's
+// max, and the nearest wins.  The object is started over by the reference's
+// traversal under the same conditions.  Clipping only (the subdivision leaf
+// keeps the reference's traversal).
 
 struct ClosestHit
 {
@@ -275,404 +428,218 @@ CGS_DEV Rings laneRings(uint32_t* lds)
                   {CGS_RING_BOT ? lane + CGS_RING_TOP * kRingStride : nullptr, CGS_RING_BOT}};
 }
 
-// ---------------------------------------------------------------------------
-// Cull-tree enumeration (cgs_cull.cpp): the elements (objects or patches)
-// whose reference leaf box a ray passes, in the tree's near-to-far order
-// ---------------------------------------------------------------------------
-
-// The cull tree's node and element records, read per lane.
-struct CullIter
+// What a lane's queries work with: its rings, region stack and its wave's
+// clip words.
+struct LaneMem
 {
-    uint32_t node, elem, elemEnd;
+    Rings rings;
+    ClipStack stack;
+    lds_u32* clip;
 };
 
-CGS_DEV bool cullable(V3 o, V3 Dinv)
+// One patch test of each lane that has one (`have`), by the chosen leaf
+// method.  Every lane of the wave calls it together.
+template<int METHOD, bool ANY>
+CGS_DEV bool leafTest(bool have, const float4* __restrict__ S, V3 o, V3 d, const TraceParams& tp, float& best, float& bu,
+                      float& bv, const LaneMem& lm, bool& overflow)
 {
-    auto ok = [](float oi, float di) { return __builtin_isfinite(oi) && __builtin_isfinite(di) && di != 0.0f; };
-    return ok(o.x, Dinv.x) && ok(o.y, Dinv.y) && ok(o.z, Dinv.z);
+    if constexpr (METHOD == Subdiv)
+        return have && subdividePatch<ANY>(S, o, d, tp.threshold, best, bu, bv, overflow);
+    else if constexpr (METHOD == ClipCapped)
+        return clipWave<ANY, true>(have, S, o, d, tp.tol2, best, bu, bv, lm.stack, lm.clip, overflow, tp.maxIters);
+    else
+        return clipWave<ANY>(have, S, o, d, kClipTol2, best, bu, bv, lm.stack, lm.clip, overflow);
 }
 
-// The next object whose reference leaf box the ray passes with entry
-// below tmax and at most lim; its entry in L0.  EMPTY at the end.
-CGS_DEV uint32_t cullNext(const SceneDev& sc, int oct, V3 o, V3 Dinv, float lim, float tmax, CullIter& it, float& L0)
+// The closest hit of each lane's ray into h (ANY: whether it has a hit, the
+// return value), for the lanes with `run`; every lane of the wave calls it
+// together.  ANY with ORIGIN: the patch `origin` is passed over and clipped
+// last.  BIG: the scene may have wide hashes and surface cull trees.
+template<int METHOD, bool ANY, bool BIG, bool ORIGIN = false>
+CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const LaneMem& lm, const V3 o, const V3 d,
+                        const float tmax, const TraceParams& tp, ClosestHit& h, bool& overflow,
+                        const OriginSkip& origin = {-1, EMPTY, false})
 {
+    h = {tmax, 0.0f, 0.0f, EMPTY, -1};
+    bool hit = false;                    // ANY: the answer
+    bool seen = false;                   // ORIGIN: the traversal reached the origin patch
+    // the objects
+    bool culled = false, tie = false;
+    float topL0 = 0.0f, hL0 = 0.0f;      // box entry of the current object, of the nearest hit's
+    Walk top {};
+    if (run)
+    {
+        const V3 Dinv {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+        culled = sc.top.cullRoot != EMPTY && cullable(o, Dinv);
+        top = culled ? cullWalk(sc.top.cullRoot) : hashWalk(sc.top.root);
+    }
+    // the current object (EMPTY: none) and its patches
+    uint32_t obj = EMPTY;
+    LocalRay lr {};
+    Walk bot {};
+    bool botCulled = false, botTie = false;
+    float botL0 = 0.0f, lL0 = 0.0f, lt = 0.0f, lu = 0.0f, lv = 0.0f;
+    uint32_t lp = EMPTY;
     while (true)
     {
-        while (it.elem < it.elemEnd)
+        uint32_t pid = EMPTY, patchBase = 0;
+        if (run)
         {
-            CGS_COUNT(kWorkCullElem);
-            const float4 a = sc.cullElems[2 * (size_t)it.elem], b = sc.cullElems[2 * (size_t)it.elem + 1];
-            it.elem++;
-            float l;
-            if (nodeIntersect<-1>(l, {a.x, a.y, a.z}, {b.x, b.y, b.z}, o, Dinv) && l < tmax && l <= lim)
+            while (true)
             {
-                L0 = l;
-                return __float_as_uint(a.w);
+                if (obj == EMPTY)
+                {
+                    const V3 Dinv {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+                    if (culled)
+                    {
+                        obj = cullNext(sc, dirOctant(Dinv), o, Dinv, ANY ? tmax : cullLimit(h.t, o), tmax, top, topL0);
+                        if (!ANY && obj == EMPTY && (tie || (h.object >= 0 && !(hL0 < h.t))))
+                        {
+                            // the reference's visit order decides
+                            culled = false;
+                            h = {tmax, 0.0f, 0.0f, EMPTY, -1};
+                            top = hashWalk(sc.top.root);
+                            continue;
+                        }
+                    }
+                    else
+                        obj = hashNext<true, true, BIG>(bvhRef(sc, sc.top), o, Dinv, ANY ? tmax : h.t, nc, lm.rings.top, top);
+                    if (obj == EMPTY)
+                    {
+                        run = false;
+                        break;
+                    }
+                    const DevObject& ob = sc.objects[obj];
+                    if (ob.surface == EMPTY)   // no geometry (empty box: only a NaN ray gets here)
+                    {
+                        obj = EMPTY;
+                        continue;
+                    }
+                    CGS_COUNT(kWorkObject);
+                    lr = toLocal(ob, o, d, tmax);
+                    const DevBVH& surf = sc.surfaces[ob.surface];
+                    botCulled = false;
+                    if constexpr (BIG && METHOD != Subdiv)
+                        botCulled = surf.cullRoot != EMPTY && cullable(lr.o, {1.0f / lr.d.x, 1.0f / lr.d.y, 1.0f / lr.d.z});
+                    bot = botCulled ? cullWalk(surf.cullRoot) : hashWalk(surf.root);
+                    lt = lr.max;
+                    lp = EMPTY;
+                    botTie = false;
+                }
+                const DevBVH& surf = sc.surfaces[sc.objects[obj].surface];
+                const V3 Dinv {1.0f / lr.d.x, 1.0f / lr.d.y, 1.0f / lr.d.z};
+                if (BIG && METHOD != Subdiv && botCulled)
+                {
+                    pid = cullNext(sc, dirOctant(Dinv), lr.o, Dinv, ANY ? lr.max : cullLimit(lt, lr.o), lr.max, bot, botL0);
+                    if (!ANY && pid == EMPTY && (botTie || (lp != EMPTY && !(lL0 < lt))))
+                    {
+                        botCulled = false;
+                        bot = hashWalk(surf.root);
+                        lt = lr.max;
+                        lp = EMPTY;
+                        continue;
+                    }
+                }
+                else
+                    pid = hashNext<CGS_BOT_OCTANTS, false, BIG>(bvhRef(sc, surf), lr.o, Dinv, ANY ? lr.max : lt,
+                                                                NodeCache {nullptr, 0}, lm.rings.bot, bot);
+                if (pid != EMPTY)
+                {
+                    if (ORIGIN && (int32_t)obj == origin.object && pid == origin.patch)
+                    {
+                        seen = true;
+                        pid = EMPTY;
+                        continue;
+                    }
+                    patchBase = surf.patchBase;
+                    break;
+                }
+                // the object is done: its hit at the world distance t / |M d|
+                if (!ANY && lp != EMPTY)
+                {
+                    const float t = lt * lr.dinv;
+                    if (t < h.t)
+                    {
+                        h = {t, lu, lv, lp, (int32_t)obj};
+                        hL0 = topL0;
+                        tie = false;
+                    }
+                    else if (t == h.t)
+                        tie = true;
+                }
+                obj = EMPTY;
             }
         }
-        if (it.node == EMPTY) return EMPTY;
-        CGS_COUNT(kWorkCullNode);
-        const float4 a = sc.cullNodes[2 * (size_t)it.node], b = sc.cullNodes[2 * (size_t)it.node + 1];
-        const uint2 l = sc.cullLinks[8 * (size_t)it.node + oct];
-        float tn;
-        const bool pass = nodeIntersect<-1>(tn, {a.x, a.y, a.z}, {b.x, b.y, b.z}, o, Dinv) && tn <= lim;
-        const uint32_t count = __float_as_uint(b.w);
-        if (pass && count)
+        const bool have = pid != EMPTY;
+        if (__ballot(have) == 0) break;
+        // test the patches: a culled surface's from the local ray's max
+        float t = ANY || botCulled ? lr.max : lt, u = 0.0f, v = 0.0f;
+        bool over = false;
+        const float4* S = sc.patches + 16 * (size_t)(have ? patchBase + pid : 0);
+        const bool f = leafTest<METHOD, ANY>(have, S, lr.o, versor3(lr.d), tp, t, u, v, lm, over);
+        if (have)
         {
-            it.elem = __float_as_uint(a.w);
-            it.elemEnd = it.elem + count;
+            if (over && botCulled)
+            {
+                // the object again, in the reference's order
+                botCulled = false;
+                bot = hashWalk(sc.surfaces[sc.objects[obj].surface].root);
+                lt = lr.max;
+                lp = EMPTY;
+            }
+            else if (over && culled)
+            {
+                // the ray again, in the reference's order
+                culled = false;
+                h = {tmax, 0.0f, 0.0f, EMPTY, -1};
+                top = hashWalk(sc.top.root);
+                obj = EMPTY;
+                seen = false;
+            }
+            else
+            {
+                if (over) overflow = true;
+                if (ANY)
+                {
+                    if (f)
+                    {
+                        hit = true;
+                        run = false;
+                    }
+                }
+                else if (f && (!botCulled || t < lt))
+                {
+                    lt = t;
+                    lu = u;
+                    lv = v;
+                    lp = pid;
+                    lL0 = botL0;
+                    botTie = false;
+                }
+                else if (f && t == lt)
+                    botTie = true;
+            }
         }
-        it.node = pass && !count ? l.x : l.y;
     }
-}
-
-// How far beyond the nearest hit so far an object's box entry may lie and
-// the object still be tested: 2^-10 of the distance plus the origin's
-// magnitude, orders of magnitude above the FP32 rounding of a hit distance
-// or a box entry.
-CGS_DEV float cullLimit(float best, float mag) { return best + (best + mag) * 0x1p-10f; }
-
-CGS_DEV int dirOctant(V3 Dinv)
-{
-    return (__builtin_signbit(Dinv.x) ? 1 : 0) | (__builtin_signbit(Dinv.y) ? 2 : 0) | (__builtin_signbit(Dinv.z) ? 4 : 0);
-}
-
-// The patches of a large surface through its cull tree: the argument of the
-// objects' enumeration (the comment above closestCulled) one level down.  A
-// patch's clip accepts candidates by the running distance only (onHit's
-// t < best), so a patch's own nearest hit does not depend on the distance
-// its test starts from; every patch whose leaf box the local ray passes near
-// or before the nearest hit so far is clipped from the local ray's max, and
-// the nearest wins.  Returns false, its outputs untouched, where the
-// reference's visit order could decide: a tie, L0_W >= t_W, a region-stack
-// overflow, a ray with a zero or non-finite component.  Clipping only (the
-// subdivision leaf keeps the reference's traversal).
-template<int METHOD>
-CGS_DEV bool surfaceClosestCulled(const SceneDev& sc, const DevBVH& surf, const LocalRay& lr, const ClipRay& cr,
-                                  const ClipStack& stk, const TraceParams& tp, float& lt, float& lu, float& lv,
-                                  uint32_t& lp, bool& hit)
-{
-    const V3 Dinv {1.0f / lr.d.x, 1.0f / lr.d.y, 1.0f / lr.d.z};
-    if (!cullable(lr.o, Dinv)) return false;
-    const int oct = dirOctant(Dinv);
-    const float mag = fmax_(__builtin_fabsf(lr.o.x), fmax_(__builtin_fabsf(lr.o.y), __builtin_fabsf(lr.o.z)));
-    float bt = lr.max, bu = 0.0f, bv = 0.0f, L0W = 0.0f, L0;
-    uint32_t bp = EMPTY, pid;
-    bool tie = false, overflow = false;
-    CullIter it {surf.cullRoot, 0u, 0u};
-    while ((pid = cullNext(sc, oct, lr.o, Dinv, cullLimit(bt, mag), lr.max, it, L0)) != EMPTY)
+    if constexpr (ORIGIN)
     {
-        const float4* S = sc.patches + 16 * (size_t)(surf.patchBase + pid);
-        float t = lr.max, u = 0.0f, v = 0.0f;
-        bool f;
-        if constexpr (METHOD == Clip)
-            f = clipPatch<false>(S, cr, kClipTol2, t, u, v, stk, overflow);
-        else
-            f = leafTest<METHOD, false>(S, cr, tp, t, u, v, stk, overflow);
-        if (overflow) return false;
-        if (!f) continue;
-        if (t < bt)
+        // the origin patch that the traversal passed over: the same local ray
+        // and patch test as the traversal's leaf
+        const bool have = seen && !hit;
+        if (__ballot(have))
         {
-            bt = t;
-            bu = u;
-            bv = v;
-            bp = pid;
-            L0W = L0;
-            tie = false;
-        }
-        else if (t == bt)
-            tie = true;
-    }
-    if (tie || (bp != EMPTY && !(L0W < bt))) return false;
-    hit = bp != EMPTY;
-    if (hit)
-    {
-        lt = bt;
-        lu = bu;
-        lv = bv;
-        lp = bp;
-    }
-    return true;
-}
-
-// A shadow ray's own surface patch, clipped last.  An any-hit answer is the
-// OR of the patch tests the traversal reaches, in whatever order, so a query
-// may pass over one patch, note that the traversal reached it (`seen`), and
-// clip it only if no other patch is hit (originAny).  A shadow ray that
-// grazes its origin patch clips it for up to thousands of passes; one that
-// another patch occludes then never does.
-struct OriginSkip
-{
-    int32_t object;
-    uint32_t patch;
-    bool seen;
-};
-
-// rt::intersect(BezierSurface, ray) through the surface's cull tree: any
-// patch whose leaf box the ray passes below the local max and that has a
-// hit, in any order (the reference's any-hit walk never narrows its limit).
-// Returns false where an overflow or the ray's components call for the
-// reference's traversal.
-template<int METHOD>
-CGS_DEV bool surfaceAnyCulled(const SceneDev& sc, const DevBVH& surf, const LocalRay& lr, const ClipRay& cr,
-                              const ClipStack& stk, const TraceParams& tp, bool& occluded, uint32_t skip = EMPTY,
-                              OriginSkip* origin = nullptr)
-{
-    const V3 Dinv {1.0f / lr.d.x, 1.0f / lr.d.y, 1.0f / lr.d.z};
-    if (!cullable(lr.o, Dinv)) return false;
-    const int oct = dirOctant(Dinv);
-    float L0;
-    uint32_t pid;
-    bool overflow = false;
-    CullIter it {surf.cullRoot, 0u, 0u};
-    while ((pid = cullNext(sc, oct, lr.o, Dinv, lr.max, lr.max, it, L0)) != EMPTY)
-    {
-        if (pid == skip)
-        {
-            origin->seen = true;
-            continue;
-        }
-        const float4* S = sc.patches + 16 * (size_t)(surf.patchBase + pid);
-        float best = lr.max, bu, bv;
-        bool f;
-        if constexpr (METHOD == Clip)
-            f = clipPatch<true>(S, cr, kClipTol2, best, bu, bv, stk, overflow);
-        else
-            f = leafTest<METHOD, true>(S, cr, tp, best, bu, bv, stk, overflow);
-        if (overflow) return false;
-        if (f)
-        {
-            occluded = true;
-            return true;
+            const float4* S = sc.patches;
+            if (have)
+            {
+                const DevObject& ob = sc.objects[origin.object];
+                lr = toLocal(ob, o, d, tmax);
+                S += 16 * (size_t)(sc.surfaces[ob.surface].patchBase + origin.patch);
+            }
+            float best = lr.max, u, v;
+            if (leafTest<METHOD, true>(have, S, lr.o, versor3(lr.d), tp, best, u, v, lm, overflow)) hit = true;
         }
     }
-    occluded = false;
-    return true;
-}
-
-// rt::intersect(BezierSurface, hit, ray) (Primitive.cu:222-248) for object
-// i, from RayTracer.cu:305-333: the object-local ray, the per-object hashed
-// traversal from t = ray.max·|M d|, and the leaf test at each patch.  On a
-// hit, t is the world distance (local t / |M d|).
-template<int METHOD, bool BIG = true>
-CGS_DEV bool objectClosest(const SceneDev& sc, const Rings& rg, uint32_t i, V3 o, V3 d, float tmax,
-                           const ClipStack& stk, bool& overflow, const TraceParams& tp, float& t, float& u, float& v,
-                           uint32_t& patch)
-{
-    const DevObject& ob = sc.objects[i];
-    if (ob.surface == EMPTY) return false;   // no geometry (empty box: only a NaN ray gets here)
-    CGS_COUNT(kWorkObject);
-    LocalRay lr = toLocal(ob, o, d, tmax);
-    const DevBVH surf = sc.surfaces[ob.surface];
-    const BVHRef b = bvhRef(sc, surf);
-    const ClipRay cr = makeClipRay(lr.o, versor3(lr.d));
-    float lt = lr.max, lu = 0.0f, lv = 0.0f;
-    uint32_t lp = EMPTY;
-    bool hit = false;
-    if constexpr (BIG && METHOD != Subdiv)
-        if (surf.cullRoot != EMPTY && surfaceClosestCulled<METHOD>(sc, surf, lr, cr, stk, tp, lt, lu, lv, lp, hit))
-        {
-            if (!hit) return false;
-            t = lt * lr.dinv;
-            u = lu;
-            v = lv;
-            patch = lp;
-            return true;
-        }
-    hit = hashIntersect<CGS_BOT_OCTANTS, false, BIG>(b, lr.o, lr.d, lt, [&](uint32_t pid) -> bool {
-        const float4* S = sc.patches + 16 * (size_t)(surf.patchBase + pid);
-        bool f;
-        // the default keeps the direct call: routing it through leafTest
-        // costs the render and trace kernels hundreds of spilled VGPRs
-        if constexpr (METHOD == Clip)
-            f = clipPatch<false>(S, cr, kClipTol2, lt, lu, lv, stk, overflow);
-        else
-            f = leafTest<METHOD, false>(S, cr, tp, lt, lu, lv, stk, overflow);
-        if (f) lp = pid;
-        return f;
-    }, NodeCache {nullptr, 0}, rg.bot);
-    if (!hit) return false;
-    t = lt * lr.dinv;
-    u = lu;
-    v = lv;
-    patch = lp;
-    return true;
-}
-
-// rt::intersect(BezierSurface, ray) (Primitive.cu:250-268) for object i.
-template<int METHOD, bool BIG = true>
-CGS_DEV bool objectAny(const SceneDev& sc, const Rings& rg, uint32_t i, V3 o, V3 d, float tmax, const ClipStack& stk,
-                       bool& overflow, const TraceParams& tp, OriginSkip* origin = nullptr)
-{
-    const DevObject& ob = sc.objects[i];
-    if (ob.surface == EMPTY) return false;   // no geometry (empty box: only a NaN ray gets here)
-    CGS_COUNT(kWorkObject);
-    LocalRay lr = toLocal(ob, o, d, tmax);
-    const DevBVH surf = sc.surfaces[ob.surface];
-    const BVHRef b = bvhRef(sc, surf);
-    const ClipRay cr = makeClipRay(lr.o, versor3(lr.d));
-    const uint32_t skip = origin && (int32_t)i == origin->object ? origin->patch : EMPTY;
-    if constexpr (BIG && METHOD != Subdiv)
-    {
-        bool occluded;
-        if (surf.cullRoot != EMPTY && surfaceAnyCulled<METHOD>(sc, surf, lr, cr, stk, tp, occluded, skip, origin))
-            return occluded;
-    }
-    return hashIntersectAny<CGS_BOT_OCTANTS, false, BIG>(b, lr.o, lr.d, lr.max, [&](uint32_t pid) -> bool {
-        if (pid == skip)
-        {
-            origin->seen = true;
-            return false;
-        }
-        const float4* S = sc.patches + 16 * (size_t)(surf.patchBase + pid);
-        float best = lr.max, bu, bv;
-        if constexpr (METHOD == Clip)
-            return clipPatch<true>(S, cr, kClipTol2, best, bu, bv, stk, overflow);
-        else
-            return leafTest<METHOD, true>(S, cr, tp, best, bu, bv, stk, overflow);
-    }, NodeCache {nullptr, 0}, rg.bot);
-}
-
-// ---------------------------------------------------------------------------
-// Object enumeration through the cull tree (cgs_cull.cpp)
-// ---------------------------------------------------------------------------
-//
-// The reference's top-level traversal reaches object X only if the ray
-// passes X's leaf box with entry L0 below the hit distance at that moment
-// (rt/BVH.h:147-266), and every ancestor box contains X's box, so it passes
-// there whenever it passes X's (the slab test is monotone in the box).
-// Each object's own result does not depend on the visit order (its traversal
-// starts from ray.max·|M d|, RayTracer.cu:311-314).  So:
-//  - any hit: the reference's answer is whether some object whose leaf box
-//    the ray passes with L0 < ray.max has a hit, in any order;
-//  - closest: enumerating every such object whose L0 is not far beyond the
-//    nearest hit found so far (a hit lies inside its object's box, up to
-//    rounding, for which the slack below leaves a wide margin) finds the
-//    nearest hit W.  The reference reaches W when L0_W < t_W (its limit is
-//    never below t_W), and then reports W unless another object has a hit at
-//    exactly t_W, where its visit order decides.
-// A lane falls back to the reference's traversal for a tie, for L0_W >= t_W,
-// for a clip-stack overflow on the way (so that overflows are reported as in
-// the reference order), and for rays on which the slab test could meet a
-// NaN (a zero or non-finite direction component, a non-finite origin).
-
-template<int METHOD, bool BIG = true>
-CGS_DEV ClosestHit closestCulled(const SceneDev& sc, const Rings& rg, V3 o, V3 d, V3 Dinv, float tmax,
-                                 const ClipStack& stk, const TraceParams& tp, bool& exact)
-{
-    ClosestHit h {tmax, 0.0f, 0.0f, EMPTY, -1};
-    const int oct = dirOctant(Dinv);
-    const float mag = fmax_(__builtin_fabsf(o.x), fmax_(__builtin_fabsf(o.y), __builtin_fabsf(o.z)));
-    float L0W = 0.0f, L0;
-    bool tie = false, overflow = false;
-    CullIter it {sc.top.cullRoot, 0u, 0u};
-    uint32_t i;
-    while ((i = cullNext(sc, oct, o, Dinv, cullLimit(h.t, mag), tmax, it, L0)) != EMPTY)
-    {
-        float t, u, v;
-        uint32_t p;
-        if (!objectClosest<METHOD, BIG>(sc, rg, i, o, d, tmax, stk, overflow, tp, t, u, v, p)) continue;
-        if (t < h.t)
-        {
-            h = {t, u, v, p, (int32_t)i};
-            L0W = L0;
-            tie = false;
-        }
-        else if (t == h.t)
-            tie = true;
-    }
-    exact = overflow || tie || (h.object >= 0 && !(L0W < h.t));
-    return h;
-}
-
-template<int METHOD, bool BIG = true>
-CGS_DEV bool anyCulled(const SceneDev& sc, const Rings& rg, V3 o, V3 d, V3 Dinv, float tmax, const ClipStack& stk,
-                       const TraceParams& tp, bool& exact, OriginSkip* origin = nullptr)
-{
-    const int oct = dirOctant(Dinv);
-    bool overflow = false;
-    CullIter it {sc.top.cullRoot, 0u, 0u};
-    float L0;
-    uint32_t i;
-    while ((i = cullNext(sc, oct, o, Dinv, tmax, tmax, it, L0)) != EMPTY)
-    {
-        const bool hit = objectAny<METHOD, BIG>(sc, rg, i, o, d, tmax, stk, overflow, tp, origin);
-        if (overflow) break;
-        if (hit) return true;
-    }
-    exact = overflow;
-    return false;
-}
-
-// Context::intersect(hit, ray) (RayTracer.cu:296-350): the nearest object
-// hit, through the cull tree where it applies, else (or where its answer
-// could depend on the visit order) by the reference's top-level traversal.
-template<int METHOD = Clip, bool BIG = true>
-CGS_DEV ClosestHit sceneClosest(const SceneDev& sc, const NodeCache& nc, const Rings& rg, V3 o, V3 d, float tmax,
-                                const ClipStack& stk, bool& overflow, const TraceParams& tp = {kClipTol2, 0x1p-4f, 0})
-{
-    if (sc.top.cullRoot != EMPTY)
-    {
-        const V3 Dinv {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
-        if (cullable(o, Dinv))
-        {
-            bool exact = false;
-            const ClosestHit h = closestCulled<METHOD, BIG>(sc, rg, o, d, Dinv, tmax, stk, tp, exact);
-            if (!exact) return h;
-        }
-    }
-    ClosestHit h {tmax, 0.0f, 0.0f, EMPTY, -1};
-    const BVHRef top = bvhRef(sc, sc.top);
-    hashIntersect<true, true, BIG>(top, o, d, h.t, [&](uint32_t i) -> bool {
-        float t, u, v;
-        uint32_t p;
-        if (objectClosest<METHOD, BIG>(sc, rg, i, o, d, tmax, stk, overflow, tp, t, u, v, p) && t < h.t)
-        {
-            h = {t, u, v, p, (int32_t)i};
-            return true;
-        }
-        return false;
-    }, nc, rg.top);
-    return h;
-}
-
-// Context::intersect(ray) (RayTracer.cu:352-383), through the cull tree
-// where it applies.  With `origin`, that patch is passed over and
-// origin->seen tells whether the traversal reached it (OriginSkip).
-template<int METHOD = Clip, bool BIG = true>
-CGS_DEV bool sceneAny(const SceneDev& sc, const NodeCache& nc, const Rings& rg, V3 o, V3 d, float tmax,
-                      const ClipStack& stk, bool& overflow, const TraceParams& tp = {kClipTol2, 0x1p-4f, 0},
-                      OriginSkip* origin = nullptr)
-{
-    if (sc.top.cullRoot != EMPTY)
-    {
-        const V3 Dinv {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
-        if (cullable(o, Dinv))
-        {
-            bool exact = false;
-            if (anyCulled<METHOD, BIG>(sc, rg, o, d, Dinv, tmax, stk, tp, exact, origin)) return true;
-            if (!exact) return false;
-            if (origin) origin->seen = false;   // the traversal below decides
-        }
-    }
-    const BVHRef top = bvhRef(sc, sc.top);
-    return hashIntersectAny<true, true, BIG>(top, o, d, tmax, [&](uint32_t i) -> bool {
-        return objectAny<METHOD, BIG>(sc, rg, i, o, d, tmax, stk, overflow, tp, origin);
-    }, nc, rg.top);
-}
-
-// The test of a shadow ray's origin patch that sceneAny passed over: object
-// i's local ray and patch test, as objectAny's leaf test.
-CGS_DEV bool originAny(const SceneDev& sc, const OriginSkip& origin, V3 o, V3 d, float tmax, const ClipStack& stk,
-                       bool& overflow)
-{
-    const DevObject& ob = sc.objects[origin.object];
-    const LocalRay lr = toLocal(ob, o, d, tmax);
-    const DevBVH surf = sc.surfaces[ob.surface];
-    const ClipRay cr = makeClipRay(lr.o, versor3(lr.d));
-    const float4* S = sc.patches + 16 * (size_t)(surf.patchBase + origin.patch);
-    float best = lr.max, bu, bv;
-    return clipPatch<true>(S, cr, kClipTol2, best, bu, bv, stk, overflow);
+    return hit;
 }
 
 // Device totals of the work events (CGS_WORK_COUNTS builds).  The sampled
@@ -717,6 +684,13 @@ CGS_DEV NodeCache stageTopLevel(const SceneDev& sc, float4* lds)
     return NodeCache {(lds_float*)(float*)lds, CGS_TOP_LDS_KEYS};
 }
 
+// A lane's query memory: its rings and its wave's clip words in LDS, its
+// region stack in `stack`.
+CGS_DEV LaneMem laneMem(uint32_t* ringLds, uint32_t* clipLds, float2* stack)
+{
+    return LaneMem {laneRings(ringLds), clipStackFor(stack, blockIdx.x * blockDim.x + threadIdx.x), waveClipWords(clipLds)};
+}
+
 // Sum of a per-lane count over the wave, added with one atomic.
 CGS_DEV void addWave(unsigned long long* ctr, unsigned long long v)
 {
@@ -745,8 +719,14 @@ CGS_DEV uint32_t nextChunk(unsigned int* counter)
 #define CGS_RENDER_WAVES 2
 #endif
 #ifndef CGS_TRACE_WAVES
-#define CGS_TRACE_WAVES 3
+#define CGS_TRACE_WAVES 2
 #endif
+
+CGS_DEV cgs_hit hitRecord(const ClosestHit& h, bool overflow)
+{
+    return {h.t, h.object < 0 ? 0.0f : h.u, h.object < 0 ? 0.0f : h.v,
+            overflow ? CGS_PATCH_OVERFLOW : (h.object < 0 ? EMPTY : h.patch)};
+}
 
 template<int METHOD, bool POLISH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_WAVES))) void kTraceClosest(SceneDev sc, Persist ps, const cgs_ray* __restrict__ rays, uint32_t n,
@@ -754,20 +734,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
                                                      unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
     __shared__ float4 topLds[4 * CGS_TOP_LDS_KEYS];
-    __shared__ uint32_t ringLds[kRingWords];
+    __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
     const NodeCache nc = stageTopLevel(sc, topLds);
-    const Rings rg = laneRings(ringLds);
-    const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl);
+    const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     unsigned long long nOverflow = 0;
     for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
     {
         const uint32_t r = base + (threadIdx.x & 63);
-        if (r >= n) continue;
+        const bool run = r < n;
         bool overflow = false;
-        const cgs_ray ray = rays[r];
-        ClosestHit h = sceneClosest<METHOD>(sc, nc, rg, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz}, ray.tmax,
-                                            stk, overflow, tp);
+        const cgs_ray ray = run ? rays[r] : cgs_ray {};
+        ClosestHit h;
+        sceneQuery<METHOD, false, true>(run, sc, nc, lm, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz}, ray.tmax, tp, h,
+                                        overflow);
+        if (!run) continue;
         if constexpr (POLISH)
             if (h.object >= 0 && !overflow)
             {
@@ -777,12 +757,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
                 polishHit64(sc.patches + 16 * (size_t)(surf.patchBase + h.patch), ob.w2l, {ray.ox, ray.oy, ray.oz},
                             {ray.dx, ray.dy, ray.dz}, h.t, h.u, h.v);
             }
-        cgs_hit out;
-        out.t = h.t;
-        out.u = h.object < 0 ? 0.0f : h.u;
-        out.v = h.object < 0 ? 0.0f : h.v;
-        out.patch = overflow ? CGS_PATCH_OVERFLOW : (h.object < 0 ? EMPTY : h.patch);
-        hits[r] = out;
+        hits[r] = hitRecord(h, overflow);
         if (objects) objects[r] = h.object;
         nOverflow += overflow;
     }
@@ -795,24 +770,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
                                                  unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
     __shared__ float4 topLds[4 * CGS_TOP_LDS_KEYS];
-    __shared__ uint32_t ringLds[kRingWords];
+    __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
     const NodeCache nc = stageTopLevel(sc, topLds);
-    const Rings rg = laneRings(ringLds);
-    const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl);
+    const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     unsigned long long nOverflow = 0;
     for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
     {
         const uint32_t r = base + (threadIdx.x & 63);
-        if (r >= n) continue;
+        const bool run = r < n;
         bool overflow = false;
-        const cgs_ray ray = rays[r];
-        bool occ = sceneAny<METHOD>(sc, nc, rg, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz}, ray.tmax, stk, overflow,
-                                    tp);
+        const cgs_ray ray = run ? rays[r] : cgs_ray {};
+        ClosestHit unused;
+        const bool occ = sceneQuery<METHOD, true, true>(run, sc, nc, lm, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz},
+                                                        ray.tmax, tp, unused, overflow);
+        if (!run) continue;
         occluded[r] = overflow ? 2u : (occ ? 1u : 0u);
         nOverflow += overflow;
     }
     addWave(overflowCount, nOverflow);
+}
+
+// The job of ray r: the last with rayBase <= r.
+template<class Job>
+CGS_DEV uint32_t jobOf(const Job* __restrict__ jobs, uint32_t njobs, uint32_t r)
+{
+    uint32_t lo = 0, hi = njobs;
+    while (hi - lo > 1)
+    {
+        const uint32_t mid = (lo + hi) / 2;
+        if (jobs[mid].rayBase <= r) lo = mid;
+        else hi = mid;
+    }
+    return lo;
 }
 
 // Batched ray queries over many resident scenes in one launch: rays of all
@@ -826,11 +815,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
     const BatchJob* __restrict__ jobs, uint32_t njobs, uint32_t total, uint32_t chunk, Persist ps,
     unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
-    const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl);
+    __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
+    const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     const NodeCache none {nullptr, 0};
-    __shared__ uint32_t ringLds[kRingWords];
-    const Rings rg = laneRings(ringLds);
     unsigned long long nOverflow = 0;
     while (true)
     {
@@ -842,43 +829,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
         for (uint32_t r0 = base; r0 < end; r0 += 64)
         {
             const uint32_t r = r0 + (threadIdx.x & 63);
-            if (r >= end) continue;
-            uint32_t lo = 0, hi = njobs;  // last job with rayBase <= r
-            while (hi - lo > 1)
-            {
-                const uint32_t mid = (lo + hi) / 2;
-                if (jobs[mid].rayBase <= r) lo = mid;
-                else hi = mid;
-            }
-            const BatchJob& J = jobs[lo];
+            const bool run = r < end;
+            const BatchJob& J = jobs[jobOf(jobs, njobs, run ? r : base)];
             const uint32_t k = r - J.rayBase;
-            const cgs_ray ray = J.rays[k];
+            const cgs_ray ray = run ? J.rays[k] : cgs_ray {};
+            const V3 o {ray.ox, ray.oy, ray.oz}, d {ray.dx, ray.dy, ray.dz};
             bool overflow = false;
-            if (J.any)
+            const bool any = run && J.any, closest = run && !J.any;
+            ClosestHit h;
+            if (__ballot(any))
             {
-                const bool occ = sceneAny<METHOD, BIG>(J.sc, none, rg, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz},
-                                                  ray.tmax, stk, overflow, tp);
-                J.occluded[k] = overflow ? 2u : (occ ? 1u : 0u);
+                const bool occ = sceneQuery<METHOD, true, BIG>(any, J.sc, none, lm, o, d, ray.tmax, tp, h, overflow);
+                if (any) J.occluded[k] = overflow ? 2u : (occ ? 1u : 0u);
             }
-            else
+            if (__ballot(closest))
             {
-                ClosestHit h = sceneClosest<METHOD, BIG>(J.sc, none, rg, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz},
-                                                    ray.tmax, stk, overflow, tp);
-                if constexpr (POLISH)
-                    if (h.object >= 0 && !overflow)
-                    {
-                        const DevObject& ob = J.sc.objects[h.object];
-                        const DevBVH surf = J.sc.surfaces[ob.surface];
-                        polishHit64(J.sc.patches + 16 * (size_t)(surf.patchBase + h.patch), ob.w2l,
-                                    {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz}, h.t, h.u, h.v);
-                    }
-                cgs_hit out;
-                out.t = h.t;
-                out.u = h.object < 0 ? 0.0f : h.u;
-                out.v = h.object < 0 ? 0.0f : h.v;
-                out.patch = overflow ? CGS_PATCH_OVERFLOW : (h.object < 0 ? EMPTY : h.patch);
-                J.hits[k] = out;
-                if (J.objects) J.objects[k] = h.object;
+                sceneQuery<METHOD, false, BIG>(closest, J.sc, none, lm, o, d, ray.tmax, tp, h, overflow);
+                if (closest)
+                {
+                    if constexpr (POLISH)
+                        if (h.object >= 0 && !overflow)
+                        {
+                            const DevObject& ob = J.sc.objects[h.object];
+                            const DevBVH surf = J.sc.surfaces[ob.surface];
+                            polishHit64(J.sc.patches + 16 * (size_t)(surf.patchBase + h.patch), ob.w2l, o, d, h.t, h.u, h.v);
+                        }
+                    J.hits[k] = hitRecord(h, overflow);
+                    if (J.objects) J.objects[k] = h.object;
+                }
             }
             nOverflow += overflow;
         }
@@ -892,18 +870,18 @@ __global__ __launch_bounds__(256) void kClipBatch(Persist ps, const cgs_ray* __r
                                                   const float4* __restrict__ patches, uint32_t n, float tol2,
                                                   cgs_hit* __restrict__ hits)
 {
-    const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl);
+    __shared__ uint32_t clipLds[kClipGroupWords];
+    const ClipStack stk = clipStackFor(ps.stack, blockIdx.x * blockDim.x + threadIdx.x);
     for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
     {
         const uint32_t r = base + (threadIdx.x & 63);
-        if (r >= n) continue;
-        const cgs_ray ray = rays[r];
+        const bool run = r < n;
+        const cgs_ray ray = run ? rays[r] : cgs_ray {};
         bool overflow = false;
-        const ClipRay cr = makeClipRay({ray.ox, ray.oy, ray.oz}, versor3({ray.dx, ray.dy, ray.dz}));
         float t = ray.tmax, u = 0.0f, v = 0.0f;
-        bool f = clipPatch<false>(patches + 16 * (size_t)r, cr, tol2, t, u, v, stk, overflow);
-        hits[r] = {t, u, v, overflow ? CGS_PATCH_OVERFLOW : (f ? 1u : EMPTY)};
+        const bool f = clipWave<false>(run, patches + 16 * (size_t)(run ? r : 0), {ray.ox, ray.oy, ray.oz},
+                                       versor3({ray.dx, ray.dy, ray.dz}), tol2, t, u, v, stk, waveClipWords(clipLds), overflow);
+        if (run) hits[r] = {t, u, v, overflow ? CGS_PATCH_OVERFLOW : (f ? 1u : EMPTY)};
     }
 }
 
@@ -1084,42 +1062,44 @@ template<bool ANY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_WAVES))) void kPick(SceneDev sc, Persist ps, const cgs_ray* __restrict__ rays, uint32_t n,
                                                             cgs_hit* __restrict__ hits, uint32_t* __restrict__ occluded)
 {
-    __shared__ uint32_t ringLds[kRingWords];
-    const Rings rg = laneRings(ringLds);
-    const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl);
+    __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
+    const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     const DevBVH surf = sc.surfaces[0];
     const BVHRef b = bvhRef(sc, surf);
     for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
     {
         const uint32_t r = base + (threadIdx.x & 63);
-        if (r >= n) continue;
-        const cgs_ray ray = rays[r];
+        bool run = r < n;
+        const cgs_ray ray = run ? rays[r] : cgs_ray {};
         const V3 o {ray.ox, ray.oy, ray.oz};
         const V3 d = versor3({ray.dx, ray.dy, ray.dz});
-        const ClipRay cr = makeClipRay(o, d);
-        bool overflow = false;
-        if (ANY)
+        const V3 Dinv {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+        bool overflow = false, hit = false;
+        float t = ray.tmax, u = 0.0f, v = 0.0f;
+        uint32_t patch = EMPTY;
+        Walk walk = hashWalk(surf.root);
+        while (true)
         {
-            const bool f = hashIntersectAny<true>(b, o, d, ray.tmax, [&](uint32_t pid) -> bool {
-                float best = __builtin_inff(), bu, bv;
-                return clipPatch<true>(sc.patches + 16 * (size_t)(surf.patchBase + pid), cr, kClipTol2, best, bu, bv, stk,
-                                       overflow);
-            }, NodeCache {nullptr, 0}, rg.bot);
-            occluded[r] = overflow ? 2u : (f ? 1u : 0u);
+            uint32_t pid = EMPTY;
+            if (run)
+            {
+                pid = hashNext<true, false, true>(b, o, Dinv, ANY ? ray.tmax : t, NodeCache {nullptr, 0}, lm.rings.bot, walk);
+                run = pid != EMPTY;
+            }
+            if (__ballot(run) == 0) break;
+            const float4* S = sc.patches + 16 * (size_t)(run ? surf.patchBase + pid : 0);
+            float inf = __builtin_inff();
+            const bool f = clipWave<ANY>(run, S, o, d, kClipTol2, ANY ? inf : t, u, v, lm.stack, lm.clip, overflow);
+            if (f)
+            {
+                patch = pid;
+                hit = true;
+                if (ANY) run = false;
+            }
         }
-        else
-        {
-            float t = ray.tmax, u = 0.0f, v = 0.0f;
-            uint32_t patch = EMPTY;
-            hashIntersect<true>(b, o, d, t, [&](uint32_t pid) -> bool {
-                const bool f = clipPatch<false>(sc.patches + 16 * (size_t)(surf.patchBase + pid), cr, kClipTol2, t, u, v,
-                                                stk, overflow);
-                if (f) patch = pid;
-                return f;
-            }, NodeCache {nullptr, 0}, rg.bot);
-            hits[r] = {t, patch == EMPTY ? 0.0f : u, patch == EMPTY ? 0.0f : v, overflow ? CGS_PATCH_OVERFLOW : patch};
-        }
+        if (r >= n) continue;
+        if (ANY) occluded[r] = overflow ? 2u : (hit ? 1u : 0u);
+        else hits[r] = {t, patch == EMPTY ? 0.0f : u, patch == EMPTY ? 0.0f : v, overflow ? CGS_PATCH_OVERFLOW : patch};
     }
 }
 
@@ -1243,81 +1223,103 @@ struct SampleState
     uint32_t seed, stream, draw;
 };
 
-// The radiance carried back along one ray: the render kernel's iterative
-// trace loop with Context::trace / miss / closestHit (RayTracer.cu:194-294,
-// 385-544): closest hit, ambient + one shadow ray per light with the PBR
-// terms, then the reflection bounce while depth remains and the attenuation
-// exceeds 2^-8.  The first segment ends at rmax, bounces at infinity.  eps is
-// read from device memory per use (the traversal loops need the registers a
-// kernel argument would hold for the whole launch).  With RECORD, the first
-// segment's hit is returned in `first`.
+// The radiance carried back along one ray of each lane with `run`: the render
+// kernel's iterative trace loop with Context::trace / miss / closestHit
+// (RayTracer.cu:194-294, 385-544): closest hit, ambient + one shadow ray per
+// light with the PBR terms, then the reflection bounce while depth remains and
+// the attenuation exceeds 2^-8.  The first segment ends at rmax, bounces at
+// infinity.  Every lane of the wave calls it together, and the wave goes
+// through each stage together (sceneQuery); a lane whose path has ended helps
+// with the others' clips.  eps is read from device memory per use (the
+// traversal loops need the registers a kernel argument would hold for the
+// whole launch).  With RECORD, the first segment's hit is returned in `first`.
 // SAMPLED: the Monte Carlo branches (RayTracer.cu:403-407,473-522): no ambient
 // term, and the bounce mirrors about a GGX microfacet normal drawn from `rs`
 // (microfacet(roughness², x, y), PBR.h:159-176) with weight mix(diffuse BRDF,
 // F(M·V) G(N·R, N·V) (M·V) / (N·V N·M), metalness); the result adds to `acc`,
 // the colour carried over from the pixel's earlier samples.
 template<bool RECORD, bool BIG = true, bool SAMPLED = false>
-CGS_DEV V3 rayRadiance(const SceneDev& sc, const NodeCache& nc, const Rings& rg, V3 ro, V3 rd, float rmax, int depth,
-                       const float* eps, const ClipStack& stk, bool& overflow, uint32_t& nShadow,
-                       uint32_t& nSecondary, ClosestHit& first, V3 acc = {0.0f, 0.0f, 0.0f},
-                       SampleState* rs = nullptr)
+CGS_DEV V3 rayRadiance(bool run, const SceneDev& sc, const NodeCache& nc, const LaneMem& lm, V3 ro, V3 rd, float rmax,
+                       int depth, const float* eps, bool& overflow, uint32_t& nShadow, uint32_t& nSecondary,
+                       ClosestHit& first, V3 acc = {0.0f, 0.0f, 0.0f}, SampleState* rs = nullptr)
 {
+    const TraceParams tp {kClipTol2, 0x1p-4f, 0};
     V3 att {1.0f, 1.0f, 1.0f};
     bool primary = true;
-    while (true)
+    while (__ballot(run))
     {
-        if (!primary) nSecondary++;
-        ClosestHit h = sceneClosest<Clip, BIG>(sc, nc, rg, ro, rd, rmax, stk, overflow);
+        if (run && !primary) nSecondary++;
+        ClosestHit h;
+        sceneQuery<Clip, false, BIG>(run, sc, nc, lm, ro, rd, rmax, tp, h, overflow);
         if (RECORD && primary) first = h;
         primary = false;
-        if (h.object < 0)
+        if (run && h.object < 0)
         {
             acc = add3(acc, mulv3({sc.background[0], sc.background[1], sc.background[2]}, att));
-            break;
+            run = false;
         }
-        const DevObject& ob = sc.objects[h.object];
-        const float4 m0 = ob.mat0, m1 = ob.mat1;
-        const float metal = m0.w, rough = m1.w;
-        const V3 spec {m1.x, m1.y, m1.z};
+        if (__ballot(run) == 0) break;
+        float metal = 0.0f, rough = 0.0f, dotNV = 0.0f;
+        V3 spec {}, diffuse {}, col {}, V {}, N {}, Pt {};
         const float invPi = 0x1.45f306p-2f; // std::numbers::inv_pi_v<float>
-        const V3 diffuse = mul3(1.0f - metal, mul3(invPi, {m0.x, m0.y, m0.z}));
-        V3 col = SAMPLED ? V3 {0.0f, 0.0f, 0.0f} : mulv3({sc.ambient[0], sc.ambient[1], sc.ambient[2]}, diffuse);
-        V3 V = neg3(rd);
-        const DevBVH surf = sc.surfaces[ob.surface];
-        V3 N = versor3(normalMat(sc.patches + 16 * (size_t)(surf.patchBase + h.patch), h.u, h.v));
-        M4 W;
-        W.c[0] = ob.w2l[0]; W.c[1] = ob.w2l[1]; W.c[2] = ob.w2l[2]; W.c[3] = ob.w2l[3];
-        N = versor3(m3tmul(W, N));
-        float dotNV = dot3(N, V);
-        if (dotNV < 0.0f)
+        if (run)
         {
-            N = neg3(N);
-            dotNV = -dotNV;
+            const DevObject& ob = sc.objects[h.object];
+            const float4 m0 = ob.mat0, m1 = ob.mat1;
+            metal = m0.w;
+            rough = m1.w;
+            spec = {m1.x, m1.y, m1.z};
+            diffuse = mul3(1.0f - metal, mul3(invPi, {m0.x, m0.y, m0.z}));
+            if (!SAMPLED) col = mulv3({sc.ambient[0], sc.ambient[1], sc.ambient[2]}, diffuse);
+            V = neg3(rd);
+            N = versor3(normalMat(sc.patches + 16 * (size_t)(sc.surfaces[ob.surface].patchBase + h.patch), h.u, h.v));
+            M4 W;
+            W.c[0] = ob.w2l[0]; W.c[1] = ob.w2l[1]; W.c[2] = ob.w2l[2]; W.c[3] = ob.w2l[3];
+            N = versor3(m3tmul(W, N));
+            dotNV = dot3(N, V);
+            if (dotNV < 0.0f)
+            {
+                N = neg3(N);
+                dotNV = -dotNV;
+            }
+            Pt = add3(ro, mul3(h.t, rd));
         }
-        V3 Pt = add3(ro, mul3(h.t, rd));
-        for (uint32_t li = 0; li < sc.nlight; li++)
+        for (uint32_t li = 0; __ballot(run && li < sc.nlight); li++)
         {
-            const DevLight lt = sc.lights[li];
-            float d;
-            V3 L;
-            if (!lightVector(d, L, Pt, lt)) continue;
-            const float dotNL = dot3(N, L);
-            if (dotNL < 1e-14f) continue;
-            nShadow++;
+            float d = 0.0f, dotNL = 0.0f;
+            V3 L {};
+            bool lit = run && li < sc.nlight;
+            if (lit)
+            {
+                lit = lightVector(d, L, Pt, sc.lights[li]);
+                if (lit)
+                {
+                    dotNL = dot3(N, L);
+                    lit = !(dotNL < 1e-14f);
+                }
+            }
+            if (__ballot(lit) == 0) continue;
+            nShadow += lit;
             // the hit's own patch last (OriginSkip): the answer is the same
-            OriginSkip origin {h.object, h.patch, false};
-            const V3 so = add3(Pt, mul3(*eps, L));
-            if (sceneAny<Clip, BIG>(sc, nc, rg, so, L, d, stk, overflow, {kClipTol2, 0x1p-4f, 0}, &origin)) continue;
-            if (origin.seen && originAny(sc, origin, so, L, d, stk, overflow)) continue;
-            V3 H = versor3(add3(L, V));
-            float dotHN = dot3(H, N);
-            float dotHL = dot3(H, L);
-            V3 I = lightColor(d, lt);
-            V3 bs = mul3(microfacet(dotNV, dotNL, dotHN, rough), schlick(spec, dotHL));
-            col = add3(col, mulv3(mul3(dotNL, I), add3(diffuse, mul3(metal, bs))));
+            V3 so {};
+            if (lit) so = add3(Pt, mul3(*eps, L));
+            ClosestHit unused;
+            const bool occluded = sceneQuery<Clip, true, BIG, true>(lit, sc, nc, lm, so, L, d, tp, unused, overflow,
+                                                                    {h.object, h.patch, false});
+            if (lit && !occluded)
+            {
+                V3 H = versor3(add3(L, V));
+                float dotHN = dot3(H, N);
+                float dotHL = dot3(H, L);
+                V3 I = lightColor(d, sc.lights[li]);
+                V3 bs = mul3(microfacet(dotNV, dotNL, dotHN, rough), schlick(spec, dotHL));
+                col = add3(col, mulv3(mul3(dotNL, I), add3(diffuse, mul3(metal, bs))));
+            }
         }
+        if (!run) continue;
         acc = add3(acc, mulv3(mul3(0x1.921fb6p+1f, col), att));
-        if (depth <= 0) break;
+        run = false;   // until the bounce is known to go on
+        if (depth <= 0) continue;
         V3 R, brdf;
         if constexpr (SAMPLED)
         {
@@ -1328,19 +1330,19 @@ CGS_DEV V3 rayRadiance(const SceneDev& sc, const NodeCache& nc, const Rings& rg,
             const float thetaM = atan2Quadrant(alpha * sqrtf(x), sqrtf(1.0f - x));
             const float phiM = 0x1.921fb6p+2f * y;   // 2π y
             const V3 ts = versor3(cross3(N, V));
-            const V3 tp = versor3(cross3(N, ts));
+            const V3 tp2 = versor3(cross3(N, ts));
             float sinT, cosT, sinP, cosP;
             sinCosAngle(thetaM, sinT, cosT);
             sinCosAngle(phiM, sinP, cosP);
-            const V3 M = versor3(add3(add3(mul3(sinT * cosP, ts), mul3(sinT * sinP, tp)), mul3(cosT, N)));
+            const V3 M = versor3(add3(add3(mul3(sinT * cosP, ts), mul3(sinT * sinP, tp2)), mul3(cosT, N)));
             const float dotMV = dot3(M, V);
             const V3 refl = schlick(spec, dotMV);
             R = sub3(neg3(V), mul3(2.0f * -dotMV, M));
             const float dotMN = dot3(M, N);
             const float dotNR = dot3(N, R);
-            if (dotNR < 1e-14f) break;
+            if (dotNR < 1e-14f) continue;
             const float g = Gsmith(dotNR, dotNV, rough) * dotMV / (dotNV * dotMN);
-            brdf = add3(mul3(1.0f - metal, mul3(invPi, {m0.x, m0.y, m0.z})), mul3(metal, mul3(g, refl)));
+            brdf = add3(diffuse, mul3(metal, mul3(g, refl)));
         }
         else
         {
@@ -1351,12 +1353,13 @@ CGS_DEV V3 rayRadiance(const SceneDev& sc, const NodeCache& nc, const Rings& rg,
             brdf = mul3(rr * rr, mul3(dotNV, add3(diffuse, mul3(metal, mul3(g, refl)))));
         }
         V3 a = mulv3(att, brdf);
-        if (max3(a) <= 0x1p-8f) break;
+        if (max3(a) <= 0x1p-8f) continue;
         ro = add3(Pt, mul3(*eps, R));
         rd = R;
         rmax = __builtin_inff();
         att = a;
         depth = depth - 1;
+        run = true;
     }
     return acc;
 }
@@ -1378,12 +1381,10 @@ template<bool BIG, bool SAMPLED = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_WAVES))) void kRender(SceneDev sc, Persist ps, const RenderArgs* ra)
 {
     __shared__ float4 topLds[4 * CGS_TOP_LDS_KEYS];
-    __shared__ uint32_t ringLds[kRingWords];
+    __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
     workBegin();
     const NodeCache nc = stageTopLevel(sc, topLds);
-    const Rings rg = laneRings(ringLds);
-    const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl);
+    const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     const uint32_t lane = threadIdx.x & 63;
     uint32_t nItems;
     {
@@ -1404,7 +1405,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
         const uint32_t tile = ra->order ? ra->order[rank] : rank;
         const unsigned long long tileStart = wall_clock64();
         const uint32_t i = (tile % tilesX) * 8 + (lane & 7), j = (tile / tilesX) * 8 + (lane >> 3);
-        if (i >= op.width || j >= op.height) continue;
+        const bool run = i < op.width && j < op.height;
         bool overflow = false;
         ClosestHit unused;
         V3 acc;
@@ -1416,7 +1417,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
             acc = {0.0f, 0.0f, 0.0f};
             for (uint32_t smp = 0; smp < n; smp++)
             {
-                nPrimary++;
+                nPrimary += run;
                 const CamDev cs = ra->cam;
                 M4 Cs;
                 Cs.c[0] = cs.c[0]; Cs.c[1] = cs.c[1]; Cs.c[2] = cs.c[2]; Cs.c[3] = cs.c[3];
@@ -1424,20 +1425,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
                 const float x = (float)i + (float)smp * nInv, y = (float)j + vdc(smp);
                 float4 P = make_float4(cs.tlx + cs.hdx * (2.0f * x), cs.tly - cs.hdy * (2.0f * y), -1.0f, 1.0f);
                 const V3 rd = versor3(sub3(project4(m4mul(Cs, P)), pos));
-                acc = rayRadiance<false, BIG, true>(sc, nc, rg, pos, rd, __builtin_inff(), ra->op.depth, &ra->op.eps, stk,
+                acc = rayRadiance<false, BIG, true>(run, sc, nc, lm, pos, rd, __builtin_inff(), ra->op.depth, &ra->op.eps,
                                                     overflow, nShadow, nSecondary, unused, acc, &rs);
             }
             acc = mul3(nInv, acc);
         }
         else
         {
-            nPrimary++;
+            nPrimary += run;
             // pixelRayDirection (RayTracer.cu:59-71)
             float4 P = make_float4(cam.tlx + cam.hdx * (2.0f * (float)i), cam.tly - cam.hdy * (2.0f * (float)j), -1.0f, 1.0f);
             const V3 rd = versor3(sub3(project4(m4mul(C, P)), camPos));
-            acc = rayRadiance<false, BIG>(sc, nc, rg, camPos, rd, __builtin_inff(), op.depth, &ra->op.eps, stk, overflow,
+            acc = rayRadiance<false, BIG>(run, sc, nc, lm, camPos, rd, __builtin_inff(), op.depth, &ra->op.eps, overflow,
                                           nShadow, nSecondary, unused);
         }
+        if (!run) continue;
         const uint32_t q = j * ra->op.width + i;
         if (float* color = ra->color)
         {
@@ -1477,16 +1479,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
     SceneDev sc0, const ShadeJob* __restrict__ jobs, uint32_t njobs, uint32_t total, uint32_t chunk, Persist ps,
     unsigned long long* __restrict__ counts)
 {
-    __shared__ uint32_t ringLds[kRingWords];
+    __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
     NodeCache nc {nullptr, 0};
     if constexpr (ONE_SCENE)
     {
         __shared__ float4 topLds[4 * CGS_TOP_LDS_KEYS];
         nc = stageTopLevel(sc0, topLds);
     }
-    const Rings rg = laneRings(ringLds);
-    const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-    const ClipStack stk = clipStackFor(ps.stack, gl);
+    const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     uint32_t nPrimary = 0, nShadow = 0, nSecondary = 0, nOverflow = 0;
     while (true)
     {
@@ -1498,40 +1498,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
         for (uint32_t r0 = base; r0 < end; r0 += 64)
         {
             const uint32_t r = r0 + (threadIdx.x & 63);
-            if (r >= end) continue;
-            uint32_t lo = 0, hi = njobs;  // last job with rayBase <= r
-            while (hi - lo > 1)
-            {
-                const uint32_t mid = (lo + hi) / 2;
-                if (jobs[mid].rayBase <= r) lo = mid;
-                else hi = mid;
-            }
-            const ShadeJob& J = jobs[lo];
+            const bool run = r < end;
+            const ShadeJob& J = jobs[jobOf(jobs, njobs, run ? r : base)];
             const uint32_t k = r - J.rayBase;
-            const cgs_ray ray = J.rays[k];
+            const cgs_ray ray = run ? J.rays[k] : cgs_ray {};
             bool overflow = false;
-            nPrimary++;
+            nPrimary += run;
             ClosestHit h;
             V3 acc;
             if constexpr (ONE_SCENE)
-                acc = rayRadiance<true>(sc0, nc, rg, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz}, ray.tmax,
-                                        J.depth, &J.eps, stk, overflow, nShadow, nSecondary, h);
+                acc = rayRadiance<true>(run, sc0, nc, lm, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz}, ray.tmax,
+                                        J.depth, &J.eps, overflow, nShadow, nSecondary, h);
             else
-                acc = rayRadiance<true>(J.sc, nc, rg, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz}, ray.tmax,
-                                        J.depth, &J.eps, stk, overflow, nShadow, nSecondary, h);
+                acc = rayRadiance<true>(run, J.sc, nc, lm, {ray.ox, ray.oy, ray.oz}, {ray.dx, ray.dy, ray.dz}, ray.tmax,
+                                        J.depth, &J.eps, overflow, nShadow, nSecondary, h);
+            if (!run) continue;
             J.color[3 * (size_t)k] = acc.x;
             J.color[3 * (size_t)k + 1] = acc.y;
             J.color[3 * (size_t)k + 2] = acc.z;
             if (uint32_t* px = J.pixels) px[k] = packSRGB(saturate(acc.x), saturate(acc.y), saturate(acc.z));
-            if (cgs_hit* hits = J.hits)
-            {
-                cgs_hit out;
-                out.t = h.t;
-                out.u = h.object < 0 ? 0.0f : h.u;
-                out.v = h.object < 0 ? 0.0f : h.v;
-                out.patch = overflow ? CGS_PATCH_OVERFLOW : (h.object < 0 ? EMPTY : h.patch);
-                hits[k] = out;
-            }
+            if (cgs_hit* hits = J.hits) hits[k] = hitRecord(h, overflow);
             if (int32_t* objects = J.objects) objects[k] = h.object;
             nOverflow += overflow;
         }
