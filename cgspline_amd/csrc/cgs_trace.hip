@@ -885,18 +885,190 @@ __global__ __launch_bounds__(256) void kClipBatch(Persist ps, const cgs_ray* __r
     }
 }
 
-__global__ __launch_bounds__(256) void kSubdivBatch(const cgs_ray* __restrict__ rays, const float4* __restrict__ patches,
-                                                    uint32_t n, float threshold, cgs_hit* __restrict__ hits)
+// Batched subdivision (Spline_Subdivision.cu:168-288): ray r against patch r,
+// `perWave` pairs to each (one-wave) workgroup.  A pair's regions depend on
+// nothing but themselves: the nearest triangle hit wins whatever the order, so
+// a wave's lanes share its pairs' regions as ClipLane's do (the oldest entry of
+// a lane that has more than one, one for one by rank; entry indices are the
+// reference's stack depths), and a pair whose order decides (two hits at
+// exactly the winning distance, or an overflow where it was shared) is
+// subdivided again unshared.  A region is small (its corners), and its net is
+// cut from the patch's each time, so any lane can take it.  With one lane per
+// pair, its stack in scratch memory and a workgroup of four waves, 30,001 pairs
+// kept half the SIMDs idle and took 1,300 us; this way 147 us.
+constexpr int kSubdivLds = 16;   // stack entries in LDS; deeper ones in scratch memory
+enum SubdivField : uint32_t
 {
-    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    const cgs_ray ray = rays[r];
-    const V3 o {ray.ox, ray.oy, ray.oz};
-    const V3 d = versor3({ray.dx, ray.dy, ray.dz});
-    float best = ray.tmax, bu = 0.0f, bv = 0.0f;
-    bool overflow = false;
-    const bool found = subdividePatch<false>(patches + 16 * (size_t)r, o, d, threshold, best, bu, bv, overflow);
-    hits[r] = {best, bu, bv, overflow ? CGS_PATCH_OVERFLOW : (found ? 1u : EMPTY)};
+    kSubOx, kSubOy, kSubOz, kSubDx, kSubDy, kSubDz, kSubPair, kSubKey, kSubTie, kSubU, kSubV, kSubFlags, kSubGiver,
+    kSubFields
+};
+
+__global__ __launch_bounds__(64) void kSubdivBatch(const cgs_ray* __restrict__ rays, const float4* __restrict__ patches,
+                                                   uint32_t n, uint32_t perWave, float threshold,
+                                                   cgs_hit* __restrict__ hits)
+{
+    __shared__ float4 stackLds[kSubdivLds * 64];
+    __shared__ uint32_t wordsLds[kSubFields * 64];
+    lds_u32* w = (lds_u32*)wordsLds;
+    const uint32_t lane = threadIdx.x, r = blockIdx.x * perWave + lane;
+    const bool mine = lane < perWave && r < n;
+    float4 deep[kSubdivStack - kSubdivLds];
+    // an entry: (umin, vmin, umax, vmax), the side in umin's sign
+    auto put = [&](int i, float4 e, bool side) {
+        e.x = __uint_as_float(__float_as_uint(e.x) | (side ? 0x80000000u : 0u));
+        if (i < kSubdivLds) stackLds[i * 64 + lane] = e;
+        else deep[i - kSubdivLds] = e;
+    };
+    float tmax = 0.0f;
+    bool todo = mine;
+    if (mine)
+    {
+        const cgs_ray ray = rays[r];
+        const V3 d = versor3({ray.dx, ray.dy, ray.dz});
+        tmax = ray.tmax;
+        w[kSubOx * 64 + lane] = __float_as_uint(ray.ox);
+        w[kSubOy * 64 + lane] = __float_as_uint(ray.oy);
+        w[kSubOz * 64 + lane] = __float_as_uint(ray.oz);
+        w[kSubDx * 64 + lane] = __float_as_uint(d.x);
+        w[kSubDy * 64 + lane] = __float_as_uint(d.y);
+        w[kSubDz * 64 + lane] = __float_as_uint(d.z);
+        w[kSubPair * 64 + lane] = r;
+    }
+    // hits lie at t > 0: none is nearer than a tmax of 0 or less or NaN
+    const uint32_t first = tmax > 0.0f ? __float_as_uint(tmax) : 0u;
+    uint32_t key = 0, flags = 0;
+    for (bool alone = false;; alone = true)
+    {
+        if (todo)
+        {
+            w[kSubKey * 64 + lane] = first;
+            w[kSubTie * 64 + lane] = 0xFFFFFFFFu;
+            w[kSubFlags * 64 + lane] = 0u;
+        }
+        int sp = 0, lo = 0;          // entries lo..sp-1 of this lane's stack
+        uint32_t own = lane;         // whose pair they belong to
+        if (todo)
+        {
+            float4 net[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) net[i] = patches[16 * (size_t)r + i];
+            V3 mn, mx;
+            projBox(net, mn, mx);
+            const V3 o {__uint_as_float(w[kSubOx * 64 + lane]), __uint_as_float(w[kSubOy * 64 + lane]),
+                        __uint_as_float(w[kSubOz * 64 + lane])};
+            const V3 d {__uint_as_float(w[kSubDx * 64 + lane]), __uint_as_float(w[kSubDy * 64 + lane]),
+                        __uint_as_float(w[kSubDz * 64 + lane])};
+            if (boxHit(mn, mx, o, d))
+            {
+                put(0, {0.0f, 0.0f, 0.5f, 1.0f}, false);
+                put(1, {0.5f, 0.0f, 1.0f, 1.0f}, false);
+                sp = 2;
+            }
+        }
+        waveOrder();
+        // ends: every lane with entries takes one region of its depth-first walk per turn
+        while (const uint64_t busy = __ballot(sp > lo))
+        {
+            if (!alone && busy != ~0ull)
+            {
+                const bool spare = sp - lo > 1 && lo < kSubdivLds;
+                if (const uint64_t give = __ballot(spare))
+                {
+                    const uint32_t rank = lanesBelow(give), idle = lanesBelow(~busy);
+                    if (spare) w[kSubGiver * 64 + rank] = lane;
+                    waveOrder();
+                    const bool take = sp == lo && idle < (uint32_t)__popcll(give);
+                    const uint32_t src = take ? w[kSubGiver * 64 + idle] : lane;
+                    const int srcLo = __shfl(lo, (int)src, 64);
+                    const uint32_t srcOwn = (uint32_t)__shfl((int)own, (int)src, 64);
+                    float4 e {};
+                    if (take) e = stackLds[srcLo * 64 + src];
+                    waveOrder();
+                    if (take)
+                    {
+                        own = srcOwn;
+                        lo = srcLo;
+                        sp = lo + 1;
+                        stackLds[lo * 64 + lane] = e;
+                        ldsOr(w + kSubFlags * 64 + own, kClipShared);
+                    }
+                    else if (spare && rank < 64u - (uint32_t)__popcll(busy))
+                        lo++;
+                    waveOrder();
+                }
+            }
+            if (sp > lo)
+            {
+                sp--;
+                float4 e = sp < kSubdivLds ? stackLds[sp * 64 + lane] : deep[sp - kSubdivLds];
+                const bool side = __builtin_signbit(e.x);
+                e.x = __builtin_fabsf(e.x);
+                const float4* S = patches + 16 * (size_t)w[kSubPair * 64 + own];
+                const V3 o {__uint_as_float(w[kSubOx * 64 + own]), __uint_as_float(w[kSubOy * 64 + own]),
+                            __uint_as_float(w[kSubOz * 64 + own])};
+                const V3 d {__uint_as_float(w[kSubDx * 64 + own]), __uint_as_float(w[kSubDy * 64 + own]),
+                            __uint_as_float(w[kSubDz * 64 + own])};
+                float4 sub[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) sub[i] = S[i];
+                subpatch4(sub, true, e.y, e.w);
+                subpatch4(sub, false, e.x, e.z);
+                V3 mn, mx;
+                projBox(sub, mn, mx);
+                if (boxHit(mn, mx, o, d))
+                {
+                    const float x = 0.5f * (e.x + e.z);
+                    const float y = 0.5f * (e.y + e.w);
+                    if ((e.z - e.x) < threshold && (e.w - e.y) < threshold)
+                    {
+                        const V3 p00 = project4(sub[0]), p10 = project4(sub[3]), p01 = project4(sub[12]),
+                                 p11 = project4(sub[15]);
+                        float t = 0.0f, t1 = 0.0f;
+                        const bool b0 = triHit(o, d, p10, p01, p00, t);
+                        const bool b1 = triHit(o, d, p01, p10, p11, t1);
+                        if (b1 && (!b0 || t1 < t)) t = t1;
+                        if (b0 || b1)
+                        {
+                            const uint32_t tb = __float_as_uint(t), old = ldsMin(w + kSubKey * 64 + own, tb);
+                            if (tb < old)
+                            {
+                                // unless another lane's hit of this turn is nearer still
+                                if (w[kSubKey * 64 + own] == tb)
+                                {
+                                    w[kSubU * 64 + own] = __float_as_uint(x);
+                                    w[kSubV * 64 + own] = __float_as_uint(y);
+                                }
+                            }
+                            else if (tb == old)
+                                ldsMin(w + kSubTie * 64 + own, tb);
+                        }
+                    }
+                    else if (sp + 2 > kSubdivStack)
+                    {
+                        ldsOr(w + kSubFlags * 64 + own, kClipOverflowed);
+                        sp = lo;
+                    }
+                    else
+                    {
+                        put(sp, side ? make_float4(e.x, e.y, x, e.w) : make_float4(e.x, e.y, e.z, y), !side);
+                        put(sp + 1, side ? make_float4(x, e.y, e.z, e.w) : make_float4(e.x, y, e.z, e.w), !side);
+                        sp += 2;
+                    }
+                }
+            }
+            waveOrder();
+        }
+        key = w[kSubKey * 64 + lane];
+        flags = w[kSubFlags * 64 + lane];
+        todo = todo && (flags & kClipShared) &&
+               ((flags & kClipOverflowed) || (key < first && w[kSubTie * 64 + lane] == key));
+        if (__ballot(todo) == 0) break;
+    }
+    if (!mine) return;
+    const bool found = key < first;
+    hits[r] = {found ? __uint_as_float(key) : tmax, found ? __uint_as_float(w[kSubU * 64 + lane]) : 0.0f,
+               found ? __uint_as_float(w[kSubV * 64 + lane]) : 0.0f,
+               (flags & kClipOverflowed) ? CGS_PATCH_OVERFLOW : (found ? 1u : EMPTY)};
 }
 
 // ---------------------------------------------------------------------------
@@ -1683,8 +1855,11 @@ hipError_t launchSubdivBatch(const cgs_ray* rays, const float* patches, uint32_t
                              hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(kSubdivBatch, dim3(blocks(n, 256)), dim3(256), 0, s, rays, (const float4*)patches, n, threshold,
-                       hits);
+    // Pairs per wave: a full wave's where they fill the chip's 2,048 resident
+    // waves, fewer below (down to 8: a pair's regions keep about 8 lanes at work)
+    const uint32_t perWave = std::clamp<uint32_t>(n / 2048u / 8u * 8u, 8u, 64u);
+    hipLaunchKernelGGL(kSubdivBatch, dim3(blocks(n, perWave)), dim3(64), 0, s, rays, (const float4*)patches, n, perWave,
+                       threshold, hits);
     return hipGetLastError();
 }
 

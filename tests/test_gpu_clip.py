@@ -1,11 +1,13 @@
-"""The batched clipper against the oracle, bit for bit: tolerances whose square
-decides convergence."""
+"""The batched per-patch kernels against the oracle, bit for bit, at the sizes
+where a wave's sharing and remainders can go wrong: tolerances whose square
+decides convergence, pairs that share a wave with none, one or many others,
+hits tied between regions, and waves of patches with a remainder."""
 from __future__ import annotations
 
 import numpy as np
 import pytest
 
-from conftest import say
+from conftest import rng, say
 from test_gpu_parity import assert_bits_equal, random_patch_pairs
 
 pytestmark = pytest.mark.gpu
@@ -24,3 +26,65 @@ def clip_equal(ctx, oracle, rays, P, tol=2.0 ** -12):
 def test_tolerances(ctx, oracle, tol):
     say("bezier_clip: tolerance", tol)
     clip_equal(ctx, oracle, *random_patch_pairs(5000, 33), tol=tol)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1000])
+def test_wave_remainders(ctx, oracle, n):
+    """Idle lanes take regions of the few busy ones (n below a wave)."""
+    say("bezier_clip, subdivision: pairs", n)
+    rays, P = random_patch_pairs(n, 40 + n)
+    clip_equal(ctx, oracle, rays, P)
+    subdivide_equal(ctx, oracle, rays, P, 2.0 ** -4)
+
+
+def subdivide_equal(ctx, oracle, rays, P, threshold):
+    g = ctx.subdivision(rays, P, threshold)
+    o, w = oracle.clip_batch(rays, P, method=1, threshold=threshold)
+    assert np.array_equal(g.view(np.uint32)[:, 3] == 1, o[:, 3] == 1)
+    assert_bits_equal(g[:, :3], o[:, :3], "t,u,v")
+
+
+def grazing_pairs(n, seed):
+    """Rays nearly in the plane of nearly flat patches: hundreds of passes over
+    as many regions, shared by the whole wave."""
+    r = rng(seed)
+    size = 8.0
+    g = np.linspace(0, size, 4)
+    P = np.zeros((n, 16, 4), np.float32)
+    P[:, :, 0], P[:, :, 1] = np.tile(g, 4), np.repeat(g, 4)
+    P[:, :, 2] = r.uniform(-1e-4, 1e-4, (n, 16))
+    P[:, :, 3] = 1.0
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, 0], rays[:, 1] = -0.2 * size, r.uniform(0.1, 0.9, n) * size
+    rays[:, 2] = r.uniform(-5e-5, 5e-5, n)
+    rays[:, 3] = np.inf
+    rays[:, 4:7] = np.stack([np.ones(n), r.uniform(-0.3, 0.3, n), r.uniform(-1e-6, 1e-6, n)], 1)
+    return rays, P
+
+
+@pytest.mark.parametrize("n", [5, 64, 200])
+def test_grazing_pairs(ctx, oracle, n):
+    say("bezier_clip, subdivision: grazing pairs", n)
+    rays, P = grazing_pairs(n, 50)
+    w = clip_equal(ctx, oracle, rays, P)
+    assert w["subdivs"] > 40 * n
+    subdivide_equal(ctx, oracle, rays, P, 2.0 ** -5)
+
+
+@pytest.mark.parametrize("threshold", [0.6, 2.0 ** -1, 2.0 ** -8])
+def test_tied_hits(ctx, oracle, threshold):
+    """Flat patches folded onto themselves (u and 1 - u at the same point):
+    every hit is found at the same distance in two regions, and the first in
+    the reference's order is reported."""
+    say("bezier_clip, subdivision: ties, threshold", threshold)
+    n = 130
+    r = rng(60)
+    P = np.zeros((n, 16, 4), np.float32)
+    P[:, :, 0] = np.tile([0.0, 1.0, 1.0, 0.0], 4)
+    P[:, :, 1] = np.repeat(np.linspace(0, 1, 4), 4)
+    P[:, :, 3] = 1.0
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, 0], rays[:, 1] = r.uniform(0.05, 0.7, n), r.uniform(0.1, 0.9, n)
+    rays[:, 2], rays[:, 3], rays[:, 6] = 2.0, np.inf, -1.0
+    clip_equal(ctx, oracle, rays, P)
+    subdivide_equal(ctx, oracle, rays, P, threshold)
