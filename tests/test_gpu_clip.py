@@ -88,3 +88,14 @@ def test_tied_hits(ctx, oracle, threshold):
     rays[:, 2], rays[:, 3], rays[:, 6] = 2.0, np.inf, -1.0
     clip_equal(ctx, oracle, rays, P)
     subdivide_equal(ctx, oracle, rays, P, threshold)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129])
+def test_subpatch_remainders(ctx, oracle, n):
+    say("subpatch", n)
+    _, P = random_patch_pairs(n, 70)
+    a = rng(71).uniform(0.0, 0.5, (n, 2)).astype(np.float32)
+    R = np.stack([a[:, 0], a[:, 0] + 0.4, a[:, 1], a[:, 1] + 0.5], 1).astype(np.float32)
+    g = ctx.subpatch(P, R)
+    o = np.stack([oracle.subpatch(P[k], *R[k]) for k in range(n)])
+    assert_bits_equal(g.reshape(n, -1), o.reshape(n, -1), "points")
