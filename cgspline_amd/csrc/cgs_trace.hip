@@ -649,12 +649,13 @@ static
 #endif
 __device__ unsigned long long g_workCounts[kWorkEvents];
 
-// Clears the workgroup's event slots (the caller then passes a barrier
-// before any event) / adds them to g_workCounts at the end of a kernel.
+// Clears the workgroup's event slots / adds them to g_workCounts at the end of
+// a kernel.
 CGS_DEV void workBegin()
 {
 #if CGS_WORK_COUNTS
     if (threadIdx.x < kWorkEvents) workSlots()[threadIdx.x] = 0;
+    __syncthreads();
 #endif
 }
 CGS_DEV void workEnd()
@@ -666,15 +667,19 @@ CGS_DEV void workEnd()
 }
 
 #ifndef CGS_TOP_LDS_KEYS
-#define CGS_TOP_LDS_KEYS 512
+#define CGS_TOP_LDS_KEYS 256
 #endif
 static_assert(CGS_TOP_LDS_KEYS <= kTopKeyCap, "top-level LDS staging beyond the key map");
 
 // Stages the top-level BVH's nodes with heap key < CGS_TOP_LDS_KEYS (its upper
-// levels, visited by nearly every ray) in LDS: 64 B per key.  512 keys (32 KiB
-// per workgroup) leave room for three resident workgroups per CU.
+// levels, visited by nearly every ray of a traversal without a cull tree) in
+// LDS: 64 B per key.  256 keys (16 KiB per workgroup): with 512 the 1M-patch
+// frame took 6.66 ms against 6.49, and three workgroups of the any-hit queries
+// would not fit a CU.  A scene with a cull tree reads that BVH only for the few
+// rays whose visit order decides, and stages nothing.
 CGS_DEV NodeCache stageTopLevel(const SceneDev& sc, float4* lds)
 {
+    if (sc.top.cullRoot != EMPTY) return NodeCache {nullptr, 0};
     for (uint32_t k = threadIdx.x; k < 4 * CGS_TOP_LDS_KEYS; k += blockDim.x)
     {
         const uint32_t node = sc.topByKey[k >> 2];
@@ -717,6 +722,13 @@ CGS_DEV uint32_t nextChunk(unsigned int* counter)
 
 #ifndef CGS_RENDER_WAVES
 #define CGS_RENDER_WAVES 2
+#endif
+// Occupancy targets of the queries (waves per SIMD).  An any-hit query keeps
+// less per lane: at three waves (168 registers, a few spilled) 777,777
+// scattered rays took 860 us against 939 at two, where closest hits of a full
+// HD view took 2.06 ms against 1.94.
+#ifndef CGS_ANY_WAVES
+#define CGS_ANY_WAVES 3
 #endif
 #ifndef CGS_TRACE_WAVES
 #define CGS_TRACE_WAVES 2
@@ -765,7 +777,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
 }
 
 template<int METHOD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_WAVES))) void kTraceAny(SceneDev sc, Persist ps, const cgs_ray* __restrict__ rays, uint32_t n,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_ANY_WAVES))) void kTraceAny(SceneDev sc, Persist ps, const cgs_ray* __restrict__ rays, uint32_t n,
                                                  uint32_t* __restrict__ occluded,
                                                  unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
