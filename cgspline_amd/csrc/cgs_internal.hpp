@@ -189,6 +189,14 @@ hipError_t launchRender(const SceneDev& sc, const PersistArgs& pa, const float* 
 // in the plain render kernels' code object it raised their register spills
 // ninefold); argsDev as filled by launchRender.
 hipError_t launchRenderSampled(const SceneDev& sc, const PersistArgs& pa, const void* argsDev, hipStream_t s);
+// The plain render's kernels for scenes of several lights (cgs_render_lights.hip):
+// from two lights on.  960x540 frames of a tea scene / 64 closed surfaces / 512
+// displaced grids, shadow rays one light after the other against from a list:
+// 1 light 2.47 / 1.81 / 2.22 against 2.78 / 1.85 / 2.30 ms; 2 lights 3.60 /
+// 2.31 / 3.06 against 3.63 / 2.03 / 2.85; 6 lights 7.33 / 5.10 / 5.68 against
+// 5.53 / 3.84 / 4.26.
+constexpr uint32_t kListLights = 2;
+hipError_t launchRenderLights(const SceneDev& sc, const PersistArgs& pa, const void* argsDev, hipStream_t s);
 // The render's work-event totals (a CGS_WORK_COUNTS=1 build; zeros
 // otherwise), kWorkEvents of them (cgs_device.hpp); cleared when `reset`.
 hipError_t workCounts(unsigned long long* out, bool reset);
