@@ -72,7 +72,8 @@ CGS_DEV uint32_t lanesBelow(uint64_t mask)
 //  - any: what a lane finds among taken regions stops that lane only, since
 //    an earlier region might still overflow; the lane that holds the first
 //    regions stops the whole pair;
-//  - an overflow anywhere in a pair that was shared.
+//  - an overflow anywhere in a pair that was shared, which ends at once for
+//    all its lanes.
 //
 // What bounds it is the instruction count of a pass, on full waves and on the
 // one lane that a wave's slowest pair would keep busy.  Convergence by squared
@@ -219,6 +220,7 @@ struct ClipLane
     CGS_DEV void pass(float tol2, uint32_t maxIters)
     {
         bool stop = false;   // ANY: this pair's test is decided
+        bool full = false;   // this lane's region stack overflowed
         if (held)
         {
             // The working patch is kept in the orientation of the current
@@ -352,7 +354,7 @@ struct ClipLane
                 else if (split && sp >= CGS_CLIP_STACK)
                 {
                     ldsOr(w + kClipFlags * 64 + own, kClipOverflowed);
-                    drop = true;
+                    drop = full = true;
                 }
                 else
                 {
@@ -443,6 +445,13 @@ struct ClipLane
                 release();
             else if (pop)
                 load(stk.entry(--sp));
+        }
+        if (__ballot(full))
+        {
+            // an overflowed pair ends for every lane at work on it: its tree can
+            // be far larger than the one path the reference follows to overflow
+            waveOrder();
+            if (held && (w[kClipFlags * 64 + own] & kClipOverflowed)) release();
         }
         if (ANY)
         {

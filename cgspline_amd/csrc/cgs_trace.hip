@@ -1057,6 +1057,7 @@ __global__ __launch_bounds__(64) void kSubdivBatch(const cgs_ray* __restrict__ r
                     waveOrder();
                 }
             }
+            bool full = false;   // this lane's stack overflowed
             if (sp > lo)
             {
                 sp--;
@@ -1107,6 +1108,7 @@ __global__ __launch_bounds__(64) void kSubdivBatch(const cgs_ray* __restrict__ r
                     {
                         ldsOr(w + kSubFlags * 64 + own, kClipOverflowed);
                         sp = lo;
+                        full = true;
                     }
                     else
                     {
@@ -1116,6 +1118,9 @@ __global__ __launch_bounds__(64) void kSubdivBatch(const cgs_ray* __restrict__ r
                     }
                 }
             }
+            waveOrder();
+            // an overflowed pair ends for every lane at work on it
+            if (__ballot(full) && (w[kSubFlags * 64 + own] & kClipOverflowed)) sp = lo;
             waveOrder();
         }
         key = w[kSubKey * 64 + lane];

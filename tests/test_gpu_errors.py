@@ -113,6 +113,39 @@ def test_clip_stack_overflow_reported(ctx, oracle):
     assert np.array_equal(g[64:][found, :3].view(np.uint32), oout[found, :3].view(np.uint32))
 
 
+@pytest.mark.parametrize("n", [1, 5, 63])
+def test_overflow_in_a_partly_idle_wave(ctx, oracle, n):
+    """The same with idle lanes beside the pairs, which share their regions:
+    an overflow ends the pair for all of them (its whole tree has 2^32
+    regions), and the pairs beside it are not disturbed."""
+    scale = 16.0
+    P = planar_patch(scale)
+    rays = np.concatenate([in_plane_rays(scale, n, 0.0), in_plane_rays(scale, n // 2, 0.05, seed=8)])
+    pats = np.repeat(P[None], rays.shape[0], 0)
+    say("kClipBatch: in-plane rays overflow in a wave with idle lanes", n)
+    g = ctx.bezier_clip(rays, pats)
+    gp = g.view(np.uint32)[:, 3]
+    assert (gp[:n] == OVERFLOW).all()
+    if n // 2:
+        o, _ = oracle.clip_batch(rays[n:], pats[n:])
+        assert np.array_equal(gp[n:] == 1, o[:, 3] == 1)
+        assert np.array_equal(g[n:, :3].view(np.uint32), o[:, :3].astype(np.float32).view(np.uint32))
+    sc = one_patch_scene(P)
+    ds = ctx.scene(sc)
+    say("scene queries: the same", n)
+    _, patch, _ = ds.trace_closest(rays)
+    assert (patch[:n] == OVERFLOW).all() and not (patch[n:] == OVERFLOW).any()
+    occ = ds.trace_any(rays)
+    assert (occ[:n] == 2).all() and (occ[n:] <= 1).all()
+
+
+def one_patch_scene(P):
+    from cgspline_amd import scenes
+    return scenes.assemble([(P, np.arange(16, dtype=np.uint32)[None])],
+                           [(0, scenes.IDENTITY16, scenes.IDENTITY16, np.array([0.5] * 6 + [0.0, 0.5], np.float32))],
+                           [scenes.point_light((8.0, 8.0, 20.0), (1.0, 1.0, 1.0))])
+
+
 def test_scene_overflow_reported(ctx, oracle):
     """The same through a one-patch scene: closest-hit patch id
     CGS_PATCH_OVERFLOW, occlusion 2, and the render's overflow counter."""
