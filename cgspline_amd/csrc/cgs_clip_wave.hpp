@@ -31,7 +31,6 @@ enum ClipField : uint32_t
     kClipTie,      // least distance accepted twice (its bits)
     kClipU, kClipV,
     kClipFlags,
-    kClipPending,  // lanes at work on the pair
     kClipGiver,
     kClipFields
 };
@@ -49,9 +48,8 @@ CGS_DEV uint32_t lanesBelow(uint64_t mask)
 // A lane's part in the clipping of its wave's (ray, patch) pairs:
 // doBezierClipping with host semantics (Spline_BezierClipping.cu:46-114,
 // 174-445), for every lane's pair at once.  start() makes a pair of the lane's
-// own current, share() and pass() are called by EVERY lane of the wave
-// together, and the pair is decided (decided()) when no lane works on it any
-// more.  With ANY a pair stops at its first accepted candidate (the caller
+// own current, and share() and pass() are called by EVERY lane of the wave
+// together until no lane has a region.  With ANY a pair stops at its first accepted candidate (the caller
 // only needs "found").  tol2 is the clipping tolerance's tolSquare: a region's
 // size is compared squared.  CAPPED (an opt-in mode with no counterpart in the
 // reference): the test stops after maxIters passes of its loop and keeps what
@@ -120,7 +118,6 @@ struct ClipLane
         w[kClipKey * 64 + lane] = firstKey(best);
         w[kClipTie * 64 + lane] = 0xFFFFFFFFu;
         w[kClipFlags * 64 + lane] = 0u;
-        w[kClipPending * 64 + lane] = 1u;
         CGS_COUNT(kWorkPatch);
         const ClipRay R = makeClipRay(o, d);
         // 0 * x is NaN for the infinities and NaN
@@ -144,9 +141,7 @@ struct ClipLane
         iters = 0;
     }
 
-    // Whether no lane works on this lane's pair any more.
-    CGS_DEV bool decided() const { return w[kClipPending * 64 + lane] == 0u; }
-    // The decided pair has to be clipped again, unshared: the order decides.
+    // The pair has to be clipped again, unshared: the order decides.
     CGS_DEV bool mustRepeat(float best) const
     {
         const uint32_t flags = w[kClipFlags * 64 + lane];
@@ -156,7 +151,7 @@ struct ClipLane
         return !ANY && key < firstKey(best) && w[kClipTie * 64 + lane] == key;
     }
     CGS_DEV bool overflowed() const { return (w[kClipFlags * 64 + lane] & kClipOverflowed) != 0; }
-    // The decided pair's answer; the nearest accepted candidate (closest)
+    // The pair's answer; the nearest accepted candidate (closest)
     CGS_DEV bool found(float best) const
     {
         return ANY ? (w[kClipFlags * 64 + lane] & kClipFound) != 0 : w[kClipKey * 64 + lane] < firstKey(best);
@@ -184,19 +179,23 @@ struct ClipLane
     {
         held = false;
         sp = lo;
-        ldsAdd(w + kClipPending * 64 + own, 0xFFFFFFFFu);
     }
 
-    // Lanes with `free` and no region take one from those that have some.
-    CGS_DEV void share(bool free)
+    // Lanes without a region take one from those that have some.
+    CGS_DEV void share()
     {
+        // An overflowed pair ends for every lane at work on it: its tree can be
+        // far larger than the one path the reference follows to overflow.  (The
+        // lane that overflowed is without a region now, so the wave gets here.)
+        if (__ballot(held && taken))
+            if (held && (w[kClipFlags * 64 + own] & kClipOverflowed)) release();
         const bool spare = held && sp > lo && (taken || !alone);
-        const uint64_t give = __ballot(spare), idle = __ballot(free && !held);
+        const uint64_t give = __ballot(spare), idle = __ballot(!held);
         if (give == 0 || idle == 0) return;
         const uint32_t rank = lanesBelow(give), idleRank = lanesBelow(idle);
         if (spare) w[kClipGiver * 64 + rank] = lane;
         waveOrder();
-        const bool take = free && !held && idleRank < (uint32_t)__popcll(give);
+        const bool take = !held && idleRank < (uint32_t)__popcll(give);
         const uint32_t src = take ? w[kClipGiver * 64 + idleRank] : lane;
         const int srcLo = __shfl(lo, (int)src, 64);
         const uint32_t srcOwn = (uint32_t)__shfl((int)own, (int)src, 64);
@@ -209,7 +208,6 @@ struct ClipLane
             own = srcOwn;
             sp = lo = srcLo;
             ldsOr(w + kClipFlags * 64 + own, kClipShared);
-            ldsAdd(w + kClipPending * 64 + own, 1u);
         }
         else if (spare && rank < (uint32_t)__popcll(idle))
             lo++;
@@ -220,7 +218,6 @@ struct ClipLane
     CGS_DEV void pass(float tol2, uint32_t maxIters)
     {
         bool stop = false;   // ANY: this pair's test is decided
-        bool full = false;   // this lane's region stack overflowed
         if (held)
         {
             // The working patch is kept in the orientation of the current
@@ -354,7 +351,7 @@ struct ClipLane
                 else if (split && sp >= CGS_CLIP_STACK)
                 {
                     ldsOr(w + kClipFlags * 64 + own, kClipOverflowed);
-                    drop = full = true;
+                    drop = true;
                 }
                 else
                 {
@@ -446,13 +443,6 @@ struct ClipLane
             else if (pop)
                 load(stk.entry(--sp));
         }
-        if (__ballot(full))
-        {
-            // an overflowed pair ends for every lane at work on it: its tree can
-            // be far larger than the one path the reference follows to overflow
-            waveOrder();
-            if (held && (w[kClipFlags * 64 + own] & kClipOverflowed)) release();
-        }
         if (ANY)
         {
             // a lane that stopped its pair is that pair's own (`own` == its lane)
@@ -481,7 +471,7 @@ CGS_DEV bool clipWave(const bool have, const float4* __restrict__ S, const V3 o,
         // ends: every held lane takes one pass of its depth-first walk per turn
         while (__ballot(c.held))
         {
-            c.share(true);
+            c.share();
             c.pass(tol2, maxIters);
         }
         todo = todo && c.mustRepeat(best);
