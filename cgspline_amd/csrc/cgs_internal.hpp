@@ -132,6 +132,7 @@ struct PersistArgs
     float2* stack;          // lanes × CGS_CLIP_STACK × 20 float2
     unsigned int* counter;  // zeroed before the launch
     uint32_t grid;
+    uint32_t chunk;         // work items a wave takes at a time (launchChunk)
 };
 
 hipError_t persistentGrid(PersistKernel k, uint32_t& blocksPerCU);

@@ -753,19 +753,27 @@ CGS_DEV void addWave(unsigned long long* ctr, unsigned long long v)
 }
 
 // Persistent launches: the grid holds exactly the resident waves; each wave
-// takes chunks of 64 work items from a counter.  `lane` indexes the region
+// takes chunks of 64 work items (fewer in a small launch) from a counter.  `lane` indexes the region
 // stack slice of this lane.
 struct Persist
 {
     float2* stack;
     unsigned int* counter;
+    uint32_t chunk;          // work items a wave takes at a time
 };
 
-CGS_DEV uint32_t nextChunk(unsigned int* counter)
+// The first of the wave's next ps.chunk work items.
+CGS_DEV uint32_t nextChunk(const Persist& ps)
 {
     uint32_t base = 0;
-    if ((threadIdx.x & 63) == 0) base = atomicAdd(counter, 64u);
+    if ((threadIdx.x & 63) == 0) base = atomicAdd(ps.counter, ps.chunk);
     return __shfl(base, 0, 64);
+}
+// Whether this lane has one of the wave's items: lane k has item base + k.
+CGS_DEV bool laneHas(const Persist& ps, uint32_t base, uint32_t n)
+{
+    const uint32_t k = threadIdx.x & 63;
+    return k < ps.chunk && base + k < n;
 }
 
 #ifndef CGS_RENDER_WAVES
@@ -798,10 +806,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
     const NodeCache nc = stageTopLevel(sc, topLds);
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     unsigned long long nOverflow = 0;
-    for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
+    for (uint32_t base = nextChunk(ps); base < n; base = nextChunk(ps))
     {
         const uint32_t r = base + (threadIdx.x & 63);
-        const bool run = r < n;
+        const bool run = laneHas(ps, base, n);
         bool overflow = false;
         const cgs_ray ray = run ? rays[r] : cgs_ray {};
         ClosestHit h;
@@ -834,10 +842,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_ANY_WAV
     const NodeCache nc = stageTopLevel(sc, topLds);
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     unsigned long long nOverflow = 0;
-    for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
+    for (uint32_t base = nextChunk(ps); base < n; base = nextChunk(ps))
     {
         const uint32_t r = base + (threadIdx.x & 63);
-        const bool run = r < n;
+        const bool run = laneHas(ps, base, n);
         bool overflow = false;
         const cgs_ray ray = run ? rays[r] : cgs_ray {};
         ClosestHit unused;
@@ -932,10 +940,10 @@ __global__ __launch_bounds__(256) void kClipBatch(Persist ps, const cgs_ray* __r
 {
     __shared__ uint32_t clipLds[kClipGroupWords];
     const ClipStack stk = clipStackFor(ps.stack, blockIdx.x * blockDim.x + threadIdx.x);
-    for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
+    for (uint32_t base = nextChunk(ps); base < n; base = nextChunk(ps))
     {
         const uint32_t r = base + (threadIdx.x & 63);
-        const bool run = r < n;
+        const bool run = laneHas(ps, base, n);
         const cgs_ray ray = run ? rays[r] : cgs_ray {};
         bool overflow = false;
         float t = ray.tmax, u = 0.0f, v = 0.0f;
@@ -1328,10 +1336,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     const DevBVH surf = sc.surfaces[0];
     const BVHRef b = bvhRef(sc, surf);
-    for (uint32_t base = nextChunk(ps.counter); base < n; base = nextChunk(ps.counter))
+    for (uint32_t base = nextChunk(ps); base < n; base = nextChunk(ps))
     {
         const uint32_t r = base + (threadIdx.x & 63);
-        bool run = r < n;
+        const bool mine = laneHas(ps, base, n);
+        bool run = mine;
         const cgs_ray ray = run ? rays[r] : cgs_ray {};
         const V3 o {ray.ox, ray.oy, ray.oz};
         const V3 d = versor3({ray.dx, ray.dy, ray.dz});
@@ -1359,7 +1368,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_W
                 if (ANY) run = false;
             }
         }
-        if (r >= n) continue;
+        if (!mine) continue;
         if (ANY) occluded[r] = overflow ? 2u : (hit ? 1u : 0u);
         else hits[r] = {t, patch == EMPTY ? 0.0f : u, patch == EMPTY ? 0.0f : v, overflow ? CGS_PATCH_OVERFLOW : patch};
     }
@@ -1764,7 +1773,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
         nItems = ((op.width + 7) / 8) * ((op.height + 7) / 8) * 64;
     }
     uint32_t nPrimary = 0, nShadow = 0, nSecondary = 0, nOverflow = 0;
-    for (uint32_t base = nextChunk(ps.counter); base < nItems; base = nextChunk(ps.counter))
+    for (uint32_t base = nextChunk(ps); base < nItems; base = nextChunk(ps))
     {
         const RenderDev op = ra->op;
         const CamDev cam = ra->cam;
@@ -1772,12 +1781,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
         M4 C;
         C.c[0] = cam.c[0]; C.c[1] = cam.c[1]; C.c[2] = cam.c[2]; C.c[3] = cam.c[3];
         const V3 camPos {cam.px, cam.py, cam.pz};
-        // one wave = one 8×8 pixel tile, taken in the order of ra->order
-        const uint32_t rank = base / 64;
+        // one wave = one 8×8 pixel tile (some of its rows in a small frame), taken
+        // in the order of ra->order
+        const uint32_t rank = base / 64, pixel = base % 64 + lane;
         const uint32_t tile = ra->order ? ra->order[rank] : rank;
         const unsigned long long tileStart = wall_clock64();
-        const uint32_t i = (tile % tilesX) * 8 + (lane & 7), j = (tile / tilesX) * 8 + (lane >> 3);
-        const bool run = i < op.width && j < op.height;
+        const uint32_t i = (tile % tilesX) * 8 + (pixel & 7), j = (tile / tilesX) * 8 + (pixel >> 3);
+        const bool run = lane < ps.chunk && i < op.width && j < op.height;
         bool overflow = false;
         ClosestHit unused;
         V3 acc;
@@ -1826,7 +1836,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
         if (uint32_t* ticks = ra->tileTicks)
         {
             const unsigned long long dt = wall_clock64() - tileStart;
-            if (lane == 0) ticks[tile] = dt > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)dt;
+            if (pixel == 0) ticks[tile] = dt > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)dt;
         }
     }
     if (unsigned long long* counts = ra->counts)
@@ -1910,7 +1920,7 @@ namespace cgs
 {
 hipError_t launchRenderLights(const SceneDev& sc, const PersistArgs& pa, const void* argsDev, hipStream_t s)
 {
-    Persist ps {pa.stack, pa.counter};
+    Persist ps {pa.stack, pa.counter, pa.chunk};
     if (sc.big)
         hipLaunchKernelGGL((kRender<true, false, true>), dim3(pa.grid), dim3(256), 0, s, sc, ps, (const RenderArgs*)argsDev);
     else
@@ -1923,7 +1933,7 @@ namespace cgs
 {
 hipError_t launchRenderSampled(const SceneDev& sc, const PersistArgs& pa, const void* argsDev, hipStream_t s)
 {
-    Persist ps {pa.stack, pa.counter};
+    Persist ps {pa.stack, pa.counter, pa.chunk};
     hipLaunchKernelGGL((kRender<true, true>), dim3(pa.grid), dim3(256), 0, s, sc, ps, (const RenderArgs*)argsDev);
     return hipGetLastError();
 }
@@ -1988,7 +1998,7 @@ hipError_t launchTraceClosest(const SceneDev& sc, const PersistArgs& pa, const c
                               int32_t* objects, unsigned long long* overflow, hipStream_t s, const TraceMode& m)
 {
     if (n == 0) return hipSuccess;
-    Persist ps {pa.stack, pa.counter};
+    Persist ps {pa.stack, pa.counter, pa.chunk};
     const TraceParams tp = traceParams(m);
 #define CGS_LAUNCH_CLOSEST(M, P) \
     hipLaunchKernelGGL((kTraceClosest<M, P>), dim3(pa.grid), dim3(256), 0, s, sc, ps, rays, n, hits, objects, overflow, tp)
@@ -2012,7 +2022,7 @@ hipError_t launchTraceAny(const SceneDev& sc, const PersistArgs& pa, const cgs_r
                           unsigned long long* overflow, hipStream_t s, const TraceMode& m)
 {
     if (n == 0) return hipSuccess;
-    Persist ps {pa.stack, pa.counter};
+    Persist ps {pa.stack, pa.counter, pa.chunk};
     const TraceParams tp = traceParams(m);
     if (m.method == CGS_METHOD_SUBDIVISION)
         hipLaunchKernelGGL((kTraceAny<Subdiv>), dim3(pa.grid), dim3(256), 0, s, sc, ps, rays, n, occluded, overflow, tp);
@@ -2028,7 +2038,7 @@ hipError_t launchTraceBatch(const BatchJob* jobs, uint32_t njobs, uint32_t total
                             const TraceMode& m, bool big)
 {
     if (total == 0) return hipSuccess;
-    Persist ps {stack, counter};
+    Persist ps {stack, counter, chunk};
     const TraceParams tp = traceParams(m);
     // the default method has a kernel without the wide-hash and surface-cull paths
     if (!big && m.method != CGS_METHOD_SUBDIVISION && !m.maxIters && m.tol == kClipTol && !m.polish)
@@ -2059,7 +2069,7 @@ hipError_t launchClipBatch(const PersistArgs& pa, const cgs_ray* rays, const flo
                            cgs_hit* hits, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    Persist ps {pa.stack, pa.counter};
+    Persist ps {pa.stack, pa.counter, pa.chunk};
     hipLaunchKernelGGL(kClipBatch, dim3(pa.grid), dim3(256), 0, s, ps, rays, (const float4*)patches, n, tolSquare(tol), hits);
     return hipGetLastError();
 }
@@ -2097,7 +2107,7 @@ hipError_t launchShade(const SceneDev* one, const ShadeJob* jobs, uint32_t njobs
                        hipStream_t s)
 {
     if (total == 0 || njobs == 0) return hipSuccess;
-    Persist ps {stack, counter};
+    Persist ps {stack, counter, chunk};
     if (one)
         hipLaunchKernelGGL(kShade<true>, dim3(grid), dim3(256), 0, s, *one, jobs, njobs, total, chunk, ps, counts);
     else
@@ -2110,7 +2120,7 @@ hipError_t launchPick(const SceneDev& sc, const PersistArgs& pa, const cgs_ray* 
                       uint32_t* occluded, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    Persist ps {pa.stack, pa.counter};
+    Persist ps {pa.stack, pa.counter, pa.chunk};
     if (occluded)
         hipLaunchKernelGGL(kPick<true>, dim3(pa.grid), dim3(256), 0, s, sc, ps, rays, n, hits, occluded);
     else
@@ -2140,7 +2150,7 @@ hipError_t launchRender(const SceneDev& sc, const PersistArgs& pa, const float* 
     // so it has been read when the call returns.
     hipError_t e = hipMemcpyAsync(argsDev, &ra, sizeof ra, hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return e;
-    Persist ps {pa.stack, pa.counter};
+    Persist ps {pa.stack, pa.counter, pa.chunk};
     if (samples > 0) return launchRenderSampled(sc, pa, argsDev, s);
     // (a counting build counts in this translation unit's kernels only)
     if (sc.nlight >= kListLights && !CGS_WORK_COUNTS) return launchRenderLights(sc, pa, argsDev, s);
