@@ -10,7 +10,7 @@
 // reference's box (the child box of its leaf, as the reference tests it) and
 // the reference's per-object traversal, and the kernels fall back to the
 // reference's traversal where the result could depend on the visit order
-// (cgs_trace.hip, sceneClosest).
+// (cgs_trace.hip, sceneQuery).
 //
 // Layout (device, 16-B aligned):
 //   nodes : 2 float4 per node: (bmin.xyz, first element as bits),
