@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include "cgs_internal.hpp"
+#include "cgs_limits.hpp"
 #include "cgs_scene_dev.hpp"
 #include "cgs_clip_wave.hpp"
 #include "cgs_sample.hpp"
@@ -1282,7 +1283,8 @@ __global__ __launch_bounds__(256) void kPatchEval(uint32_t kind, const float4* _
 // again for most of its sixteen points once a CU's waves held more than its
 // 32-KiB L1.  A padded row of 17 points per patch spreads the lanes' 16-byte
 // accesses over the banks.  Bound by memory: 300,001 patches (528 bytes each)
-// took 46 us (3.4 TB/s) that way, 38 us (4.2 TB/s) this way.
+// took 46 us (3.4 TB/s) that way, 38 us (4.2 TB/s) this way.  Calls of few
+// patches (subpatchPerLane) are latency: the way through LDS adds to it.
 __global__ __launch_bounds__(64) void kSubpatch(const float4* __restrict__ patches, const float4* __restrict__ ranges,
                                                 uint32_t n, float4* __restrict__ out)
 {
@@ -1315,6 +1317,23 @@ __global__ __launch_bounds__(64) void kSubpatch(const float4* __restrict__ patch
 #pragma unroll
     for (uint32_t k = 0; k < 16; k++)
         if (k * 64 + lane < points) to[k * 64 + lane] = lds[(k * 4 + (lane >> 4)) * 17 + (lane & 15)];
+}
+
+// The same with each lane moving its own patch.
+__global__ __launch_bounds__(64) void kSubpatchFew(const float4* __restrict__ patches, const float4* __restrict__ ranges,
+                                                   uint32_t n, float4* __restrict__ out)
+{
+    const uint32_t r = blockIdx.x * 64 + threadIdx.x;
+    if (r >= n) return;
+    const float4* S = patches + 16 * (size_t)r;
+    float4 p[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) p[i] = S[i];
+    const float4 g = ranges[r];
+    subpatch4(p, true, g.z, g.w);
+    subpatch4(p, false, g.x, g.y);
+#pragma unroll
+    for (int i = 0; i < 16; i++) out[16 * (size_t)r + i] = p[i];
 }
 #endif // !CGS_SAMPLED_TU && !CGS_LIGHTS_TU
 
@@ -2097,8 +2116,8 @@ hipError_t launchPatchEval(uint32_t kind, const float* patches, const float* uv,
 hipError_t launchSubpatch(const float* patches, const float* ranges, uint32_t n, float* out, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(kSubpatch, dim3(blocks(n, 64)), dim3(64), 0, s, (const float4*)patches, (const float4*)ranges,
-                       n, (float4*)out);
+    hipLaunchKernelGGL(subpatchPerLane(n) ? kSubpatchFew : kSubpatch, dim3(blocks(n, 64)), dim3(64), 0, s,
+                       (const float4*)patches, (const float4*)ranges, n, (float4*)out);
     return hipGetLastError();
 }
 

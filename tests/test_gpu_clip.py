@@ -99,3 +99,10 @@ def test_subpatch_remainders(ctx, oracle, n):
     g = ctx.subpatch(P, R)
     o = np.stack([oracle.subpatch(P[k], *R[k]) for k in range(n)])
     assert_bits_equal(g.reshape(n, -1), o.reshape(n, -1), "points")
+
+
+@pytest.mark.parametrize("n", [100, 32767, 32768, 32769, 33001])
+def test_subpatch_at_the_kernel_switch(ctx, oracle, n):
+    """Per lane up to 32,768 patches, through LDS above."""
+    say("subpatch", n)
+    test_subpatch_remainders(ctx, oracle, n)

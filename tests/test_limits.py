@@ -48,3 +48,18 @@ def test_counter_guard(tmp_path):
     subprocess.run(["g++", "-std=c++20", "-O1", "-I", inc, str(src), "-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout
+
+
+def evaluate(tmp_path, expr):
+    """An expression over cgs_limits.hpp's rules, as an integer."""
+    src = tmp_path / "rule.cpp"
+    src.write_text('#include <cstdio>\n#include "cgs_limits.hpp"\nusing namespace cgs;\n'
+                   f'int main() {{ std::printf("%llu\\n", (unsigned long long)({expr})); }}\n')
+    inc = os.path.join(conftest.ROOT, "cgspline_amd", "csrc")
+    subprocess.run(["g++", "-std=c++20", "-I", inc, str(src), "-o", str(tmp_path / "rule")], check=True)
+    return int(subprocess.run([str(tmp_path / "rule")], stdout=subprocess.PIPE, text=True, check=True).stdout)
+
+
+def test_few_subpatches_are_moved_per_lane(tmp_path):
+    assert evaluate(tmp_path, "subpatchPerLane(1) && subpatchPerLane(100) && subpatchPerLane(32768)")
+    assert not evaluate(tmp_path, "subpatchPerLane(32769) || subpatchPerLane(300001)")
