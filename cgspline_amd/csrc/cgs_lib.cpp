@@ -117,19 +117,6 @@ struct cgs_ctx
     std::mutex mu;
 };
 
-// Work items that a wave of a persistent launch of `grid` workgroups takes at a
-// time: 64, one per lane, and fewer (down to 8, a power of two) where that
-// still gives every wave some.  A wave waits for its slowest item, and its
-// lanes without one share the others' clips: a 64-ray pick took 71 us this way
-// and 91 us in one wave, 5,000 shaded rays 640 and 1,408 us, a 200x150 frame of
-// 19 lights 3.7 and 10.3 ms, a 256x256 one-light frame 305 and 336 us.
-static uint32_t launchChunk(uint64_t items, uint32_t grid)
-{
-    uint32_t chunk = 64;
-    while (chunk > 8 && items <= (uint64_t)grid * 4 * (chunk / 2)) chunk /= 2;
-    return chunk;
-}
-
 // Grid, stack slice and zeroed work counter for one persistent launch over
 // `items` work items.  The caller holds ctx->mu, launches the kernel on `s`
 // and then calls persistEnd.  The counter grows by at most 64 per wave fetch past
@@ -160,8 +147,8 @@ static cgs_status persistArgs(cgs_ctx* ctx, PersistKernel k, hipStream_t s, uint
     }
     pa.stack = ctx->dStack;
     pa.counter = ctx->dCounters + ki;
-    pa.grid = ctx->grid[ki];
-    pa.chunk = launchChunk(items, pa.grid);
+    pa.chunk = launchChunk(items, ctx->grid[ki]);
+    pa.grid = launchGrid(items, ctx->grid[ki], pa.chunk);
     if (ctx->persistLaunched) HIP_TRY(hipStreamWaitEvent(s, ctx->persistDone, 0));
     HIP_TRY(launchFill(pa.counter, 0u, 1, s));
     return CGS_OK;
@@ -1621,8 +1608,8 @@ static cgs_status traceBatch(cgs_ctx* ctx, const cgs_batch_job* jobs, uint32_t n
     if ((st = persistArgs(ctx, PersistKernel::Batch, s, total, pa)) != CGS_OK) return st;
     HIP_TRY(hipMemcpyAsync(ctx->batchTable.p, table.data(), table.size() * sizeof(BatchJob), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s)); // the host table is released on return
-    HIP_TRY(launchTraceBatch(ctx->batchTable.as<BatchJob>(), (uint32_t)table.size(), total, chunk, pa.stack, pa.counter, grid,
-                             ctx->dOverflow, s, mode, anyBig(table)));
+    HIP_TRY(launchTraceBatch(ctx->batchTable.as<BatchJob>(), (uint32_t)table.size(), total, chunk, pa.stack, pa.counter,
+                             launchGrid(total, grid, chunk), ctx->dOverflow, s, mode, anyBig(table)));
     HIP_TRY(hipEventRecord(ctx->batchDone, s));
     ctx->batchLaunched = true;
     return persistEnd(ctx, s);
@@ -1679,7 +1666,8 @@ cgs_status cgs_batch_create(cgs_ctx* ctx, const cgs_batch_job* jobs, uint32_t nj
     if (e == hipSuccess) e = launchFill(b->counter.as<uint32_t>(), 0u, 1, cs);
     if (e == hipSuccess)
         e = launchTraceBatch(b->table.as<BatchJob>(), (uint32_t)table.size(), total, ctx->batchChunk,
-                             b->stack.as<float2>(), b->counter.as<unsigned int>(), grid,
+                             b->stack.as<float2>(), b->counter.as<unsigned int>(),
+                             launchGrid(total, grid, ctx->batchChunk),
                              b->overflow.as<unsigned long long>(), cs, ctx->batchMode, anyBig(table));
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(cs, &g);
@@ -2246,8 +2234,8 @@ struct cgs_server
             bool big = false;
             for (size_t k = 0; k < nTrace; k++) big |= jt[k].sc.big != 0;
             if ((e = launchTraceBatch(sl.table.as<BatchJob>(), (uint32_t)nTrace, traceRays, chunk, sl.stack.as<float2>(),
-                                      sl.counter.as<unsigned int>(), grid, sl.overflow.as<unsigned long long>(),
-                                      sl.stream, TraceMode {}, big)) != hipSuccess)
+                                      sl.counter.as<unsigned int>(), launchGrid(traceRays, grid, chunk),
+                                      sl.overflow.as<unsigned long long>(), sl.stream, TraceMode {}, big)) != hipSuccess)
                 return e;
         }
         if (nShade)
@@ -2256,8 +2244,8 @@ struct cgs_server
                                     sl.stream)) != hipSuccess)
                 return e;
             if ((e = launchShade(nullptr, sl.shadeTable.as<ShadeJob>(), (uint32_t)nShade, shadeRays, chunk,
-                                 sl.stack.as<float2>(), sl.counter.as<unsigned int>() + 1, shadeGrid, nullptr,
-                                 sl.stream)) != hipSuccess)
+                                 sl.stack.as<float2>(), sl.counter.as<unsigned int>() + 1,
+                                 launchGrid(shadeRays, shadeGrid, chunk), nullptr, sl.stream)) != hipSuccess)
                 return e;
         }
         if ((e = hipMemcpyAsync(sl.hOut.p, sl.out.p, outBytes, hipMemcpyDeviceToHost, sl.stream)) != hipSuccess) return e;

@@ -63,3 +63,17 @@ def evaluate(tmp_path, expr):
 def test_few_subpatches_are_moved_per_lane(tmp_path):
     assert evaluate(tmp_path, "subpatchPerLane(1) && subpatchPerLane(100) && subpatchPerLane(32768)")
     assert not evaluate(tmp_path, "subpatchPerLane(32769) || subpatchPerLane(300001)")
+
+
+def test_launches_hold_no_workgroups_without_work(tmp_path):
+    """The workgroups of a persistent launch: those that some item reaches."""
+    for items, grid, want in [(0, 768, 1), (1, 768, 1), (64, 768, 2), (64, 512, 2), (65, 768, 3), (3000, 768, 94),
+                              (24_576, 768, 768), (24_577, 768, 385), (200_000, 768, 768), (2 ** 32 - 200_000, 768, 768)]:
+        chunk = evaluate(tmp_path, f"launchChunk({items}ull, {grid})")
+        got = evaluate(tmp_path, f"launchGrid({items}ull, {grid}, {chunk})")
+        assert got == want, (items, grid, chunk, got)
+        assert 4 * got * chunk >= min(items, 4 * grid * chunk)      # every item is reached
+        assert got == 1 or 4 * (got - 1) * chunk < items            # by every workgroup
+    # a batch's chunk is the caller's
+    assert evaluate(tmp_path, "launchGrid(20000, 768, 4096)") == 2
+    assert evaluate(tmp_path, "launchGrid(1ull << 30, 768, 64)") == 768
