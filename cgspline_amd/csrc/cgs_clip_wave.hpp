@@ -175,6 +175,23 @@ struct ClipLane
         vside = r3.x != 0.0f;
     }
 
+    // The current region's points are not needed any more.  Without these empty
+    // definitions they count as live until the next region replaces them, also
+    // through the evaluation of a candidate (16 points of the patch), as a second
+    // copy beside the other lanes': a pick took 227 registers, 172 with them, and
+    // at three waves per SIMD (168) spilled 182, now 5.
+    CGS_DEV void forget()
+    {
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+        {
+            asm("" : "=v"(p[i].x));
+            asm("" : "=v"(p[i].y));
+        }
+#endif
+    }
+
     CGS_DEV void release()
     {
         held = false;
@@ -248,6 +265,7 @@ struct ClipLane
                 at[0] = {mn.x + c.x * sz.x, mn.y + c.y * sz.y};
                 cand[1] = triangleOrigin(c, p[15], c03, c30);
                 at[1] = {mx.x - c.x * sz.x, mx.y - c.y * sz.y};
+                forget();
 #pragma unroll 1
                 for (int k = 0; k < 2; k++)
                 {
@@ -347,11 +365,13 @@ struct ClipLane
                 {
                     CGS_COUNT(kWorkPrune);
                     pop = true;
+                    forget();
                 }
                 else if (split && sp >= CGS_CLIP_STACK)
                 {
                     ldsOr(w + kClipFlags * 64 + own, kClipOverflowed);
                     drop = true;
+                    forget();
                 }
                 else
                 {

@@ -1651,6 +1651,7 @@ cgs_status cgs_batch_create(cgs_ctx* ctx, const cgs_batch_job* jobs, uint32_t nj
     if ((st = buildBatchJobs(ctx, jobs, njobs, ctx->batchChunk, grid, table, total)) != CGS_OK) return st;
     auto b = std::make_unique<cgs_batch>();
     b->ctx = ctx;
+    grid = launchGrid(total, grid, ctx->batchChunk);
     const uint32_t lanes = grid * 256;
     HIP_TRY(b->table.alloc(std::max<size_t>(1, table.size()) * sizeof(BatchJob)));
     HIP_TRY(b->counter.alloc(256));
@@ -1666,8 +1667,7 @@ cgs_status cgs_batch_create(cgs_ctx* ctx, const cgs_batch_job* jobs, uint32_t nj
     if (e == hipSuccess) e = launchFill(b->counter.as<uint32_t>(), 0u, 1, cs);
     if (e == hipSuccess)
         e = launchTraceBatch(b->table.as<BatchJob>(), (uint32_t)table.size(), total, ctx->batchChunk,
-                             b->stack.as<float2>(), b->counter.as<unsigned int>(),
-                             launchGrid(total, grid, ctx->batchChunk),
+                             b->stack.as<float2>(), b->counter.as<unsigned int>(), grid,
                              b->overflow.as<unsigned long long>(), cs, ctx->batchMode, anyBig(table));
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(cs, &g);

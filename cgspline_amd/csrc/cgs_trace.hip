@@ -780,15 +780,24 @@ CGS_DEV bool laneHas(const Persist& ps, uint32_t base, uint32_t n)
 #ifndef CGS_RENDER_WAVES
 #define CGS_RENDER_WAVES 2
 #endif
-// Occupancy targets of the queries (waves per SIMD).  An any-hit query keeps
-// less per lane: at three waves (168 registers, a few spilled) 777,777
-// scattered rays took 860 us against 939 at two, where closest hits of a full
-// HD view took 2.06 ms against 1.94.
+// Occupancy targets of the queries (waves per SIMD).  Three (168 registers)
+// where a launch holds scattered rays, whose walks wait for memory: 200,000
+// picks on 1,600 patches take 308 us (closest) and 283 (any) against 351 and 337
+// at two, a batch of 64 scenes (17M rays, half of them scattered) 6.2 ms against
+// 7.1, 777,777 scattered any-hit rays 826 us.  Closest hits stay at two: 700,000
+// camera rays take 782 us against 844 at three, where 49 registers spill;
+// 700,000 scattered ones take 964 against 912.
 #ifndef CGS_ANY_WAVES
 #define CGS_ANY_WAVES 3
 #endif
-#ifndef CGS_TRACE_WAVES
-#define CGS_TRACE_WAVES 2
+#ifndef CGS_BATCH_WAVES
+#define CGS_BATCH_WAVES 3
+#endif
+#ifndef CGS_PICK_WAVES
+#define CGS_PICK_WAVES 3
+#endif
+#ifndef CGS_CLOSEST_WAVES
+#define CGS_CLOSEST_WAVES 2
 #endif
 
 CGS_DEV cgs_hit hitRecord(const ClosestHit& h, bool overflow)
@@ -798,7 +807,7 @@ CGS_DEV cgs_hit hitRecord(const ClosestHit& h, bool overflow)
 }
 
 template<int METHOD, bool POLISH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_WAVES))) void kTraceClosest(SceneDev sc, Persist ps, const cgs_ray* __restrict__ rays, uint32_t n,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_CLOSEST_WAVES))) void kTraceClosest(SceneDev sc, Persist ps, const cgs_ray* __restrict__ rays, uint32_t n,
                                                      cgs_hit* __restrict__ hits, int32_t* __restrict__ objects,
                                                      unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
@@ -880,7 +889,7 @@ CGS_DEV uint32_t jobOf(const Job* __restrict__ jobs, uint32_t njobs, uint32_t r)
 // the jobs' first ray numbers and runs the same per-ray query as
 // kTraceClosest / kTraceAny, with the same leaf methods and polish.
 template<int METHOD, bool POLISH, bool BIG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_WAVES))) void kTraceBatch(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_BATCH_WAVES))) void kTraceBatch(
     const BatchJob* __restrict__ jobs, uint32_t njobs, uint32_t total, uint32_t chunk, Persist ps,
     unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
@@ -1348,7 +1357,7 @@ __global__ __launch_bounds__(64) void kSubpatchFew(const float4* __restrict__ pa
 // (PatchBVH.cpp:93-94), so a patch whose box the traversal reaches within
 // ray.tmax counts with a hit at any distance in front.
 template<bool ANY>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_TRACE_WAVES))) void kPick(SceneDev sc, Persist ps, const cgs_ray* __restrict__ rays, uint32_t n,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_PICK_WAVES))) void kPick(SceneDev sc, Persist ps, const cgs_ray* __restrict__ rays, uint32_t n,
                                                             cgs_hit* __restrict__ hits, uint32_t* __restrict__ occluded)
 {
     __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
