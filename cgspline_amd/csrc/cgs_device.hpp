@@ -469,20 +469,35 @@ CGS_DEV uint32_t fastmod(uint32_t x, const FastMod& f)
     return (uint32_t)__umul64hi(low, (uint64_t)f.d);
 }
 
+struct DevBVH
+{
+    uint32_t root;        // absolute node offset of the root
+    uint32_t displBase;   // offset into displ
+    uint32_t tableBase;   // offset into tables
+    uint32_t A, B, mask;
+    uint32_t T;           // table size
+    uint32_t patchBase;   // first patch of the surface (surfaces only)
+    uint64_t Tm;          // fastmod multiplier for T
+    uint32_t finiteBoxes; // 1: every child box of an inner node is finite
+    uint32_t wide;        // 1: hashed with the wide family (exact arithmetic)
+    uint32_t cullRoot;    // root of its cull tree in the scene's cull arrays, or EMPTY
+    uint32_t pad[3];
+};
+static_assert(sizeof(DevBVH) == 64, "DevBVH layout");
+
 // One BVH with its perfect hash, as laid out in device memory.  Node and
-// table entries are absolute offsets into the scene's node array.
+// table entries are absolute offsets into the scene's node array.  The hash
+// parameters stay in the BVH's record, read by a lookup only: a traversal is
+// taken up again after every patch test, and with the parameters read there
+// each time a wave's chain of dependent loads grew by two.
 struct BVHRef
 {
     const float4* __restrict__ nodes;    // 4 float4 (64 B) per node
     const uint32_t* __restrict__ indices;
-    const uint32_t* __restrict__ table;
-    const uint32_t* __restrict__ displ;
-    uint32_t root;                       // absolute node offset of the root
-    uint32_t A, B, mask;
-    FastMod T;
+    const uint32_t* __restrict__ tables; // of all the scene's BVHs
+    const uint32_t* __restrict__ displs;
+    const DevBVH* __restrict__ record;
     uint32_t nodeCount;                  // size of `nodes`, bounds table lookups
-    uint32_t finiteBoxes;                // 1: every child box of an inner node is finite
-    uint32_t wide;                       // 1: the wide hash family (exact arithmetic)
 };
 
 struct NodeBoxes
@@ -614,25 +629,31 @@ CGS_DEV NodeBoxes loadNodeCached(const BVHRef& b, const NodeCache& nc, uint32_t 
     return LOW ? loadNodeLow(b.nodes, node) : loadNode(b.nodes, node);
 }
 
-// PerfectHashFunction::hash (PerfectHashFunction.h:58-63): 32-bit
-// arithmetic, or for a BVH hashed with the wide family the same function in
-// exact arithmetic, (A·(k mod T) + B + D) mod T.
+// The table's node for a key: PerfectHashFunction::hash
+// (PerfectHashFunction.h:58-63) in 32-bit arithmetic, or for a BVH hashed with
+// the wide family the same function in exact arithmetic,
+// (A·(k mod T) + B + D) mod T.
 template<bool BIG = true>
-CGS_DEV uint32_t hashKey(const BVHRef& b, uint32_t key)
+CGS_DEV uint32_t hashedNode(const BVHRef& b, uint32_t key)
 {
-    if (BIG && b.wide)
+    const DevBVH& h = *b.record;
+    const FastMod T {h.Tm, h.T};
+    const uint32_t displ = b.displs[h.displBase + (key & h.mask)];
+    uint32_t slot;
+    if (BIG && h.wide)
     {
         // x mod T through a double quotient: x < 2^63 and T < 2^31, so the
         // quotient is off by at most one and one correction each way is exact
-        const uint64_t x = (uint64_t)b.A * fastmod(key, b.T) + b.B + b.displ[key & b.mask];
-        const double q = __builtin_floor((double)x / (double)b.T.d);
-        int64_t r = (int64_t)x - (int64_t)q * (int64_t)b.T.d;
-        r += r < 0 ? (int64_t)b.T.d : 0;
-        r -= r >= (int64_t)b.T.d ? (int64_t)b.T.d : 0;
-        return (uint32_t)r;
+        const uint64_t x = (uint64_t)h.A * fastmod(key, T) + h.B + displ;
+        const double q = __builtin_floor((double)x / (double)T.d);
+        int64_t r = (int64_t)x - (int64_t)q * (int64_t)T.d;
+        r += r < 0 ? (int64_t)T.d : 0;
+        r -= r >= (int64_t)T.d ? (int64_t)T.d : 0;
+        slot = (uint32_t)r;
     }
-    uint32_t x = b.A * key + b.B + b.displ[key & b.mask];
-    return fastmod(x, b.T);
+    else
+        slot = fastmod(h.A * key + h.B + displ, T);
+    return b.tables[h.tableBase + slot];
 }
 
 // Node indices of a traversal's postponed siblings, kept per lane in LDS so
@@ -709,7 +730,7 @@ CGS_DEV bool ascend(const BVHRef& b, const NodeCache& nc, const SiblingRing& rin
     if (st.rs.pop(ring, st.node)) return true;
     if (st.key < nc.keys) return true;    // staged in LDS: read by key, no lookup
     CGS_COUNT(kWorkProbe);
-    st.node = b.table[hashKey<BIG>(b, st.key)];
+    st.node = hashedNode<BIG>(b, st.key);
     return st.node < b.nodeCount;
 }
 

@@ -24,22 +24,6 @@
 namespace cgs
 {
 
-struct DevBVH
-{
-    uint32_t root;        // absolute node offset of the root
-    uint32_t displBase;   // offset into displ
-    uint32_t tableBase;   // offset into tables
-    uint32_t A, B, mask;
-    uint32_t T;           // table size
-    uint32_t patchBase;   // first patch of the surface (surfaces only)
-    uint64_t Tm;          // fastmod multiplier for T
-    uint32_t finiteBoxes; // 1: every child box of an inner node is finite
-    uint32_t wide;        // 1: hashed with the wide family (exact arithmetic)
-    uint32_t cullRoot;    // root of its cull tree in the scene's cull arrays, or EMPTY
-    uint32_t pad[3];
-};
-static_assert(sizeof(DevBVH) == 64, "DevBVH layout");
-
 struct DevObject
 {
     float4 w2l[4];        // world→local, column-major
@@ -115,22 +99,9 @@ struct ShadeJob
     int32_t depth;
 };
 
-CGS_DEV BVHRef bvhRef(const SceneDev& sc, const DevBVH& d)
+CGS_DEV BVHRef bvhRef(const SceneDev& sc, const DevBVH* record)
 {
-    BVHRef b;
-    b.nodes = sc.nodes;
-    b.indices = sc.indices;
-    b.table = sc.tables + d.tableBase;
-    b.displ = sc.displ + d.displBase;
-    b.root = d.root;
-    b.A = d.A;
-    b.B = d.B;
-    b.mask = d.mask;
-    b.T = {d.Tm, d.T};
-    b.nodeCount = sc.nodeCount;
-    b.finiteBoxes = d.finiteBoxes;
-    b.wide = d.wide;
-    return b;
+    return {sc.nodes, sc.indices, sc.tables, sc.displ, record, sc.nodeCount};
 }
 
 } // namespace cgs

@@ -304,7 +304,7 @@ template<bool OCTANTS, bool LOW, bool BIG>
 CGS_DEV uint32_t hashNext(const BVHRef& b, V3 o, V3 Dinv, float limit, const NodeCache& nc, const SiblingRing& ring,
                           Walk& it)
 {
-    const int oct = OCTANTS ? waveOctant(o, Dinv, b.finiteBoxes) : -1;
+    const int oct = OCTANTS ? waveOctant(o, Dinv, b.record->finiteBoxes) : -1;
     while (true)
     {
         if (it.leaf != EMPTY)
@@ -365,6 +365,13 @@ struct OriginSkip
 // With the test inside each lane's own traversal loops 11 of 64 lanes were
 // active on the 1M-patch frame, and a lane whose ray grazes a patch for
 // thousands of passes held its wave alone.
+//
+// Lanes on the reference's top-level traversal (rays with a zero direction
+// component, as all of an orthographic view have that looks along an axis
+// plane, and restarted ones) wait for each other before the next object.  That
+// traversal reads about twice as many nodes as the cull tree's, and with lanes in
+// different objects each round of a wave pays for it: 1M parallel rays through
+// 2,048 grids took 5.5 ms (closest) and 4.9 (any hit) that way, 3.1 and 2.5 this.
 //
 // Objects through the cull tree.  The reference's top-level traversal reaches
 // object X only if the ray passes X's leaf box with entry L0 below the hit
@@ -488,8 +495,8 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
         culled = sc.top.cullRoot != EMPTY && cullable(o, Dinv);
         top = culled ? cullWalk(sc.top.cullRoot) : hashWalk(sc.top.root);
     }
-    // the current object (EMPTY: none) and its patches
-    uint32_t obj = EMPTY;
+    // the current object (EMPTY: none), its surface and its patches
+    uint32_t obj = EMPTY, surface = EMPTY, patchBase = 0;
     LocalRay lr {};
     Walk bot {};
     bool botCulled = false, botTie = false;
@@ -497,8 +504,10 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
     uint32_t lp = EMPTY;
     while (true)
     {
-        uint32_t pid = EMPTY, patchBase = 0;
-        if (run || (LIST && open))
+        uint32_t pid = EMPTY;
+        // lanes on the reference's top-level traversal take their next objects together
+        const bool inside = __ballot(run && !culled && obj != EMPTY) != 0;
+        if (run ? culled || obj != EMPTY || !inside : LIST && open)
         {
             while (true)
             {
@@ -531,7 +540,7 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
                         }
                     }
                     else
-                        obj = hashNext<true, true, BIG>(bvhRef(sc, sc.top), o, Dinv, ANY ? tmax : h.t, nc, lm.rings.top, top);
+                        obj = hashNext<true, true, BIG>(bvhRef(sc, &sc.top), o, Dinv, ANY ? tmax : h.t, nc, lm.rings.top, top);
                     if (LIST && obj == EMPTY && seen)
                     {
                         // the origin patch that the traversal passed over: the same
@@ -559,7 +568,9 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
                     }
                     CGS_COUNT(kWorkObject);
                     lr = toLocal(ob, o, d, tmax);
-                    const DevBVH& surf = sc.surfaces[ob.surface];
+                    surface = ob.surface;
+                    const DevBVH& surf = sc.surfaces[surface];
+                    patchBase = surf.patchBase;
                     botCulled = false;
                     if constexpr (BIG && METHOD != Subdiv)
                         botCulled = surf.cullRoot != EMPTY && cullable(lr.o, {1.0f / lr.d.x, 1.0f / lr.d.y, 1.0f / lr.d.z});
@@ -568,7 +579,6 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
                     lp = EMPTY;
                     botTie = false;
                 }
-                const DevBVH& surf = sc.surfaces[sc.objects[obj].surface];
                 const V3 Dinv {1.0f / lr.d.x, 1.0f / lr.d.y, 1.0f / lr.d.z};
                 if (BIG && METHOD != Subdiv && botCulled)
                 {
@@ -576,14 +586,14 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
                     if (!ANY && pid == EMPTY && (botTie || (lp != EMPTY && !(lL0 < lt))))
                     {
                         botCulled = false;
-                        bot = hashWalk(surf.root);
+                        bot = hashWalk(sc.surfaces[surface].root);
                         lt = lr.max;
                         lp = EMPTY;
                         continue;
                     }
                 }
                 else
-                    pid = hashNext<CGS_BOT_OCTANTS, false, BIG>(bvhRef(sc, surf), lr.o, Dinv, ANY ? lr.max : lt,
+                    pid = hashNext<CGS_BOT_OCTANTS, false, BIG>(bvhRef(sc, sc.surfaces + surface), lr.o, Dinv, ANY ? lr.max : lt,
                                                                 NodeCache {nullptr, 0}, lm.rings.bot, bot);
                 if (pid != EMPTY)
                 {
@@ -593,7 +603,6 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
                         pid = EMPTY;
                         continue;
                     }
-                    patchBase = surf.patchBase;
                     break;
                 }
                 // the object is done: its hit at the world distance t / |M d|
@@ -610,10 +619,16 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
                         tie = true;
                 }
                 obj = EMPTY;
+                if (!culled) break;
             }
         }
+        // ends: a round moves every lane that does not wait, and while lanes wait others are inside objects
         const bool have = pid != EMPTY;
-        if (__ballot(have) == 0) break;
+        if (__ballot(have) == 0)
+        {
+            if (__ballot(run)) continue;
+            break;
+        }
         // test the patches: a culled surface's from the local ray's max
         float t = ANY || botCulled ? lr.max : lt, u = 0.0f, v = 0.0f;
         bool over = false;
@@ -630,7 +645,7 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
             {
                 // the object again, in the reference's order
                 botCulled = false;
-                bot = hashWalk(sc.surfaces[sc.objects[obj].surface].root);
+                bot = hashWalk(sc.surfaces[surface].root);
                 lt = lr.max;
                 lp = EMPTY;
             }
@@ -723,11 +738,16 @@ static_assert(CGS_TOP_LDS_KEYS <= kTopKeyCap, "top-level LDS staging beyond the 
 // levels, visited by nearly every ray of a traversal without a cull tree) in
 // LDS: 64 B per key.  256 keys (16 KiB per workgroup): with 512 the 1M-patch
 // frame took 6.66 ms against 6.49, and three workgroups of the any-hit queries
-// would not fit a CU.  A scene with a cull tree reads that BVH only for the few
-// rays whose visit order decides, and stages nothing.
+// would not fit a CU.  In a scene with a cull tree only rays with a zero
+// direction component and the few whose visit order decides read that BVH: ray
+// and shading queries stage it there too (ALWAYS; parallel rays through 256
+// grids take 837 and 729 us staged, 888 and 789 not), renders, whose camera rays
+// have such a component in a column or two, do not (a 640x480 frame takes 2.23 ms
+// staged, 2.12 not).
+template<bool ALWAYS>
 CGS_DEV NodeCache stageTopLevel(const SceneDev& sc, float4* lds)
 {
-    if (sc.top.cullRoot != EMPTY) return NodeCache {nullptr, 0};
+    if (!ALWAYS && sc.top.cullRoot != EMPTY) return NodeCache {nullptr, 0};
     for (uint32_t k = threadIdx.x; k < 4 * CGS_TOP_LDS_KEYS; k += blockDim.x)
     {
         const uint32_t node = sc.topByKey[k >> 2];
@@ -813,7 +833,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_CLOSEST
 {
     __shared__ float4 topLds[4 * CGS_TOP_LDS_KEYS];
     __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
-    const NodeCache nc = stageTopLevel(sc, topLds);
+    const NodeCache nc = stageTopLevel<true>(sc, topLds);
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     unsigned long long nOverflow = 0;
     for (uint32_t base = nextChunk(ps); base < n; base = nextChunk(ps))
@@ -849,7 +869,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_ANY_WAV
 {
     __shared__ float4 topLds[4 * CGS_TOP_LDS_KEYS];
     __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
-    const NodeCache nc = stageTopLevel(sc, topLds);
+    const NodeCache nc = stageTopLevel<true>(sc, topLds);
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     unsigned long long nOverflow = 0;
     for (uint32_t base = nextChunk(ps); base < n; base = nextChunk(ps))
@@ -1362,8 +1382,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_PICK_WA
 {
     __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
-    const DevBVH surf = sc.surfaces[0];
-    const BVHRef b = bvhRef(sc, surf);
+    const DevBVH& surf = sc.surfaces[0];
+    const BVHRef b = bvhRef(sc, &surf);
     for (uint32_t base = nextChunk(ps); base < n; base = nextChunk(ps))
     {
         const uint32_t r = base + (threadIdx.x & 63);
@@ -1787,7 +1807,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
     __shared__ float4 topLds[4 * CGS_TOP_LDS_KEYS];
     __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
     workBegin();
-    const NodeCache nc = stageTopLevel(sc, topLds);
+    const NodeCache nc = stageTopLevel<false>(sc, topLds);
     LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     if constexpr (LIGHTS)
     {
@@ -1894,7 +1914,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
     if constexpr (ONE_SCENE)
     {
         __shared__ float4 topLds[4 * CGS_TOP_LDS_KEYS];
-        nc = stageTopLevel(sc0, topLds);
+        nc = stageTopLevel<true>(sc0, topLds);
     }
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     uint32_t nPrimary = 0, nShadow = 0, nSecondary = 0, nOverflow = 0;
