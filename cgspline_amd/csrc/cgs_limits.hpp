@@ -45,6 +45,14 @@ inline uint32_t launchGrid(uint64_t items, uint32_t grid, uint32_t chunk)
     return need >= grid ? grid : need ? (uint32_t)need : 1u;
 }
 
+// Whether a batched launch of `rays` rays takes the kernels of two waves per SIMD
+// rather than three: up to ten rays for each lane of two waves on the 256 CUs.
+// Then most waves hold the launch's camera rays, whose clips the spills of three
+// waves slow down; above, the scattered rays' walks need the third.  Two against
+// three: 150,000 rays 249 and 267 us, 660,000 387 and 424, 1.0M 434-491 and
+// 447-514, 1.9M 807-998 and 772-932, 3.4M 1,070 and 1,025, 17M 7.1 and 6.3 ms.
+inline bool batchAtTwoWaves(uint64_t rays) { return rays <= 10ull * 256 * 512; }
+
 // Whether a sub-patch call of n patches has each lane move its own patch
 // (kSubpatchFew) rather than a wave move its 64 through LDS (kSubpatch): up to
 // two waves per CU of 256, whose patches (16 KiB a wave) its 32-KiB L1 holds.

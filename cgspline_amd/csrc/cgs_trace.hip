@@ -802,9 +802,9 @@ CGS_DEV bool laneHas(const Persist& ps, uint32_t base, uint32_t n)
 #endif
 // Occupancy targets of the queries (waves per SIMD).  Three (168 registers)
 // where a launch holds scattered rays, whose walks wait for memory: 200,000
-// picks on 1,600 patches take 308 us (closest) and 283 (any) against 351 and 337
-// at two, a batch of 64 scenes (17M rays, half of them scattered) 6.2 ms against
-// 7.1, 777,777 scattered any-hit rays 826 us.  Closest hits stay at two: 700,000
+// picks on 1,600 patches take 308 us (closest) and 287 (any) against 351 and 337
+// at two, a batch of 64 scenes (17M rays, half of them scattered) 6.3 ms against
+// 7.1 (smaller batches: batchAtTwoWaves), 777,777 scattered any-hit rays 820 us.  Closest hits stay at two: 700,000
 // camera rays take 782 us against 844 at three, where 49 registers spill;
 // 700,000 scattered ones take 964 against 912.
 #ifndef CGS_ANY_WAVES
@@ -908,8 +908,8 @@ CGS_DEV uint32_t jobOf(const Job* __restrict__ jobs, uint32_t njobs, uint32_t r)
 // without a launch per scene.  Each lane finds its job by binary search over
 // the jobs' first ray numbers and runs the same per-ray query as
 // kTraceClosest / kTraceAny, with the same leaf methods and polish.
-template<int METHOD, bool POLISH, bool BIG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_BATCH_WAVES))) void kTraceBatch(
+template<int METHOD, bool POLISH, bool BIG, int WAVES = CGS_BATCH_WAVES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void kTraceBatch(
     const BatchJob* __restrict__ jobs, uint32_t njobs, uint32_t total, uint32_t chunk, Persist ps,
     unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
@@ -2088,11 +2088,14 @@ hipError_t launchTraceBatch(const BatchJob* jobs, uint32_t njobs, uint32_t total
     if (total == 0) return hipSuccess;
     Persist ps {stack, counter, chunk};
     const TraceParams tp = traceParams(m);
-    // the default method has a kernel without the wide-hash and surface-cull paths
-    if (!big && m.method != CGS_METHOD_SUBDIVISION && !m.maxIters && m.tol == kClipTol && !m.polish)
+    if (m.method != CGS_METHOD_SUBDIVISION && !m.maxIters && m.tol == kClipTol && !m.polish)
     {
-        hipLaunchKernelGGL((kTraceBatch<Clip, false, false>), dim3(grid), dim3(256), 0, s, jobs, njobs, total, chunk, ps,
-                           overflow, tp);
+        // the default method has kernels without the wide-hash and surface-cull
+        // paths, and both with a form for launches of few rays
+        if (batchAtTwoWaves(total)) grid = std::min(grid, 2u * 256u);
+        const auto kernel = batchAtTwoWaves(total) ? (big ? kTraceBatch<Clip, false, true, 2> : kTraceBatch<Clip, false, false, 2>)
+                                                   : (big ? kTraceBatch<Clip, false, true> : kTraceBatch<Clip, false, false>);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, jobs, njobs, total, chunk, ps, overflow, tp);
         return hipGetLastError();
     }
 #define CGS_LAUNCH_BATCH(M, P) \
@@ -2107,8 +2110,7 @@ hipError_t launchTraceBatch(const BatchJob* jobs, uint32_t njobs, uint32_t total
         if (m.polish) CGS_LAUNCH_BATCH(ClipCapped, true);
         else CGS_LAUNCH_BATCH(ClipCapped, false);
     }
-    else if (m.polish) CGS_LAUNCH_BATCH(Clip, true);
-    else CGS_LAUNCH_BATCH(Clip, false);
+    else CGS_LAUNCH_BATCH(Clip, true);
 #undef CGS_LAUNCH_BATCH
     return hipGetLastError();
 }

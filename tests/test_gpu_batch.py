@@ -154,3 +154,42 @@ def test_batch_rejects_bad_jobs(ctx, small_batch):
     assert e.value.status == 1
     with pytest.raises(cgs.CgsError):
         ctx.set_batch_config(100, 0)
+
+
+@pytest.mark.parametrize("total", [10 * 256 * 512, 10 * 256 * 512 + 1])
+@pytest.mark.parametrize("big", [False, True])
+def test_batch_at_the_kernel_switch(ctx, c2_small, c3_small, grazing, big, total):
+    """Launches of few and of many rays use kernels of their own, each with and
+    without the paths for large surfaces: hits equal the separate queries'."""
+    import cgspline_amd as cgs
+    from cgspline_amd import scenes
+    say("batch at the kernel switch: rays", total, "large surface", big)
+    jobs, left = [], total
+    for k, wl in enumerate((c2_small, c3_small, grazing if big else c2_small)):
+        n = left if k == 2 else 400_001
+        left -= n
+        rays = scenes.camera_rays(wl.camera)
+        ds = ctx.scene(wl.scene)
+        assert not big or k < 2 or ds.bvh_culled(0)
+        if k == 1:
+            want = (ds.trace_any(rays),)
+        else:
+            tuv, patch, obj = ds.trace_closest(rays)
+            want = (np.concatenate([tuv.view(np.uint32), patch[:, None].astype(np.uint32)], 1), obj)
+        at = np.arange(n) % rays.shape[0]
+        job = dict(scene=ds, rays=cgs.DeviceArray.from_host(ctx, np.ascontiguousarray(rays[at])), n=n)
+        if k == 1:
+            job.update(any=True, occluded=cgs.DeviceArray(ctx, 4 * n))
+        else:
+            job.update(hits=cgs.DeviceArray(ctx, 16 * n), objects=cgs.DeviceArray(ctx, 4 * n))
+        jobs.append((job, want, at))
+    ctx.trace_batch([j for j, _, _ in jobs])
+    ctx.sync()
+    for job, want, at in jobs:
+        n = job["n"]
+        if "occluded" in job:
+            assert np.array_equal(job["occluded"].to_host(np.uint32, (n,)), want[0][at])
+        else:
+            assert np.array_equal(job["hits"].to_host(np.uint32, (n, 4)), want[0][at])
+            assert np.array_equal(job["objects"].to_host(np.int32, (n,)), want[1][at])
+        job["scene"].destroy()

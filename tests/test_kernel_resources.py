@@ -45,8 +45,18 @@ def kernels(tmp_path_factory):
 # clip; more than about a hundred are spilled in the loop over a clip's passes.
 @pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
 @pytest.mark.parametrize("name, spills", [("5kPickILb0E", 8), ("5kPickILb1E", 8), ("9kTraceAnyILi0E", 40),
-                                          ("11kTraceBatchILi0ELb0ELb0E", 80), ("11kTraceBatchILi0ELb0ELb1E", 100)])
+                                          ("11kTraceBatchILi0ELb0ELb0ELi3E", 80),
+                                          ("11kTraceBatchILi0ELb0ELb1ELi3E", 100)])
 def test_three_waves_per_simd(kernels, name, spills):
     k = [v for n, v in kernels.items() if n.startswith("_ZN3cgs" + name)]
     assert len(k) == 1
     assert k[0]["vgpr"] <= 512 // 3 // 8 * 8 and k[0]["spill"] <= spills, k
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+@pytest.mark.parametrize("name", ["11kTraceBatchILi0ELb0ELb0ELi2E", "11kTraceBatchILi0ELb0ELb1ELi2E", "13kTraceClosestILi0ELb0E",
+                                  "7kRenderILb0ELb0ELb0E", "7kRenderILb1ELb0ELb0E"])
+def test_two_waves_per_simd_without_spills(kernels, name):
+    k = [v for n, v in kernels.items() if n.startswith("_ZN3cgs" + name)]
+    assert len(k) == 1
+    assert k[0]["vgpr"] <= 256 and k[0]["spill"] == 0, k

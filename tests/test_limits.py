@@ -77,3 +77,8 @@ def test_launches_hold_no_workgroups_without_work(tmp_path):
     # a batch's chunk is the caller's
     assert evaluate(tmp_path, "launchGrid(20000, 768, 4096)") == 2
     assert evaluate(tmp_path, "launchGrid(1ull << 30, 768, 64)") == 768
+
+
+def test_small_batches_run_at_two_waves(tmp_path):
+    assert evaluate(tmp_path, "batchAtTwoWaves(1) && batchAtTwoWaves(655360) && batchAtTwoWaves(1310720)")
+    assert not evaluate(tmp_path, "batchAtTwoWaves(1310721) || batchAtTwoWaves(1ull << 24)")
