@@ -205,7 +205,7 @@ struct ClipLane
         // far larger than the one path the reference follows to overflow.  (The
         // lane that overflowed is without a region now, so the wave gets here.)
         if (__ballot(held && taken))
-            if (held && (w[kClipFlags * 64 + own] & kClipOverflowed)) release();
+            if (held && (ldsLoad(w + kClipFlags * 64 + own) & kClipOverflowed)) release();
         const bool spare = held && sp > lo && (taken || !alone);
         const uint64_t give = __ballot(spare), idle = __ballot(!held);
         if (give == 0 || idle == 0) return;
@@ -297,7 +297,7 @@ struct ClipLane
                         if (tb < old)
                         {
                             // unless another lane's candidate of this turn is nearer still
-                            if (w[kClipKey * 64 + own] == tb)
+                            if (ldsLoad(w + kClipKey * 64 + own) == tb)
                             {
                                 w[kClipU * 64 + own] = __float_as_uint(eu);
                                 w[kClipV * 64 + own] = __float_as_uint(ev);

@@ -677,6 +677,14 @@ CGS_DEV uint32_t ldsMin(lds_u32* p, uint32_t v)
 {
     return __hip_atomic_fetch_min(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
+// A word that other lanes of the wave change in the same turn.  Atomic like the
+// changes: a plain load could be given a lane's own result of an earlier ldsMin,
+// and the lane with the least value is only found by what the word holds after
+// all lanes' (they run in step).
+CGS_DEV uint32_t ldsLoad(const lds_u32* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
 constexpr uint32_t kRingStride = 256;   // threads per workgroup: slot k of a lane is base[k * 256]
 
 struct SiblingRing

@@ -1132,7 +1132,7 @@ __global__ __launch_bounds__(64) void kSubdivBatch(const cgs_ray* __restrict__ r
                             if (tb < old)
                             {
                                 // unless another lane's hit of this turn is nearer still
-                                if (w[kSubKey * 64 + own] == tb)
+                                if (ldsLoad(w + kSubKey * 64 + own) == tb)
                                 {
                                     w[kSubU * 64 + own] = __float_as_uint(x);
                                     w[kSubV * 64 + own] = __float_as_uint(y);
@@ -1158,7 +1158,7 @@ __global__ __launch_bounds__(64) void kSubdivBatch(const cgs_ray* __restrict__ r
             }
             waveOrder();
             // an overflowed pair ends for every lane at work on it
-            if (__ballot(full) && (w[kSubFlags * 64 + own] & kClipOverflowed)) sp = lo;
+            if (__ballot(full) && (ldsLoad(w + kSubFlags * 64 + own) & kClipOverflowed)) sp = lo;
             waveOrder();
         }
         key = w[kSubKey * 64 + lane];

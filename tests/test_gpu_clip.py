@@ -90,6 +90,22 @@ def test_tied_hits(ctx, oracle, threshold):
     subdivide_equal(ctx, oracle, rays, P, threshold)
 
 
+@pytest.mark.parametrize("n", [1, 7, 64, 300])
+def test_many_hits_of_one_pair(ctx, oracle, n):
+    """Tangled nets that a ray crosses several times: lanes at work on one pair
+    find candidates in the same turn, and the nearest one's (u, v) is kept."""
+    say("bezier_clip, subdivision: tangled nets", n)
+    r = rng(90 + n)
+    P = np.ones((n, 16, 4), np.float32)
+    P[:, :, :3] = r.uniform(0.0, 1.0, (n, 16, 3))
+    o, to = r.uniform(-1.0, 2.0, (n, 3)), r.uniform(0.35, 0.65, (n, 3))
+    o[:, 2] = 3.0
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, :3], rays[:, 3], rays[:, 4:7] = o, np.inf, (to - o) / np.linalg.norm(to - o, axis=1, keepdims=True)
+    clip_equal(ctx, oracle, rays, P)
+    subdivide_equal(ctx, oracle, rays, P, 2.0 ** -5)
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 129])
 def test_subpatch_remainders(ctx, oracle, n):
     say("subpatch", n)
