@@ -4,7 +4,9 @@ The work of a launch is fixed by event counts of the deterministic algorithm
 (node visits, hash probes, leaf visits, patch tests, clip iterations by kind,
 onHit evaluations, rays), not by hardware counters.  The GPU path executes the
 same per-ray algorithm bit for bit, so the counts the CPU oracle reports for
-a workload are the GPU launch's counts.
+a workload are the GPU launch's counts of rays, and of events up to the cull
+trees, the order in which a wave's lanes share a pair's regions, and the pairs
+clipped a second time because that order decides (the library counts its own).
 
 Bytes per unit (the layout the kernels read; every fetch counted as if it
 missed in cache — the "algorithmic" traffic):
@@ -17,8 +19,8 @@ missed in cache — the "algorithmic" traffic):
   surface record)
 * per pixel written: 4 B (packed frame), +12 B if the float colour is written
 
-FP32 operations per unit (add/sub/mul/min/max/compare = 1, div/sqrt = 1),
-counted from the kernels' source:
+FP32 operations per unit of the reference algorithm (add/sub/mul/min/max/compare
+= 1, div/sqrt = 1):
 
 * inner node visit: 2 slab tests × 3 axes × (2 sub + 2 mul + 2 select +
   2 compare) + 6 = 54
@@ -59,14 +61,26 @@ GPU_EVENTS = ("cullNodes", "cullElems", "nodes", "hashProbes", "leaves", "patchT
 # the direction's transform and normalisation (15 + 10) and the clipping
 # frame (2 cross products and versors, ≈ 40): ≈ 100.
 F_CULL, F_OBJECT = 27, 100
+
+# Per event of the library's own clipping pass (cgs_clip_wave.hpp, ClipLane),
+# which computes the reference's results with fewer operations: squared sizes
+# instead of two square roots, and one de Casteljau step for both halves of a
+# split.  A pass up to its hull: tolerance 12 + line 14 + distances 48 + envelope
+# 24 + hull edges 7 x 19 + 11 + widening and its compares 7 = 249; a clip adds the
+# region 6 and eight slices 4 + 8 x 36, a split the region 2 and eight halvings
+# 8 x 18; a converged region is the tolerance 12 + two triangle tests 2 x 22 + the
+# two candidates' parameters 8; a projection adds 65 for its test of finite points.
+L_PROJ, L_CLIP, L_SPLIT, L_PRUNE, L_CONVERGED = 313, 547, 395, 249, 64
 B_CULL_NODE, B_CULL_ELEM = 40, 32
 
 
 def flops_of_counts(c: dict) -> float:
-    """FP32 operations of a launch from the library's own event counts."""
-    return (F_CULL * (c["cullNodes"] + c["cullElems"]) + F_NODE * c["nodes"] + F_PROJ * c["patchTests"]
-            + F_CLIP * c["clips"] + F_SUBDIV * c["splits"] + F_PRUNE * c["prunes"]
-            + F_CONVERGED * c["converged"] + F_ONHIT * c["onHits"] + F_OBJECT * c["objects"])
+    """FP32 operations of a launch from the library's own event counts: what it
+    executed, passes over regions past an any-hit pair's first hit and pairs
+    clipped a second time among them."""
+    return (F_CULL * (c["cullNodes"] + c["cullElems"]) + F_NODE * c["nodes"] + L_PROJ * c["patchTests"]
+            + L_CLIP * c["clips"] + L_SPLIT * c["splits"] + L_PRUNE * c["prunes"]
+            + L_CONVERGED * c["converged"] + F_ONHIT * c["onHits"] + F_OBJECT * c["objects"])
 
 
 def bytes_of_counts(c: dict, pixels: int, color: bool = False) -> float:
