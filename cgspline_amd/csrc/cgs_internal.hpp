@@ -201,6 +201,9 @@ hipError_t launchRenderLights(const SceneDev& sc, const PersistArgs& pa, const v
 // The render's work-event totals (a CGS_WORK_COUNTS=1 build; zeros
 // otherwise), kWorkEvents of them (cgs_device.hpp); cleared when `reset`.
 hipError_t workCounts(unsigned long long* out, bool reset);
+// ... added to `out`, of the several-lights and the sampled renders' kernels.
+hipError_t workCountsLights(unsigned long long* out, bool reset);
+hipError_t workCountsSampled(unsigned long long* out, bool reset);
 // order[0..n) = the tiles 0..n-1, longest `ticks` first.
 hipError_t launchTileOrder(const uint32_t* ticks, uint32_t n, uint32_t* order, hipStream_t s);
 

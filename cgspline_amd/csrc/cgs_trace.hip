@@ -705,12 +705,9 @@ CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const
     return hit;
 }
 
-// Device totals of the work events (CGS_WORK_COUNTS builds).  The other
-// renders' translation units keep copies of their own, which nothing reads.
-#if CGS_SAMPLED_TU || CGS_LIGHTS_TU
-static
-#endif
-__device__ unsigned long long g_workCounts[kWorkEvents];
+// Device totals of the work events (CGS_WORK_COUNTS builds), one set for the
+// kernels of each translation unit; workCounts adds them up.
+static __device__ unsigned long long g_workCounts[kWorkEvents];
 
 // Clears the workgroup's event slots / adds them to g_workCounts at the end of
 // a kernel.
@@ -1963,9 +1960,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
 
 } // namespace cgs
 
+namespace cgs
+{
+// Adds this translation unit's work-event totals to `out` and clears them when
+// `reset`.
+static hipError_t addWorkCounts(unsigned long long* out, bool reset)
+{
+    unsigned long long own[kWorkEvents];
+    const hipError_t e = hipMemcpyFromSymbol(own, HIP_SYMBOL(g_workCounts), sizeof own);
+    if (e != hipSuccess) return e;
+    for (int k = 0; k < kWorkEvents; k++) out[k] += own[k];
+    if (!reset) return hipSuccess;
+    const unsigned long long zero[kWorkEvents] = {};
+    return hipMemcpyToSymbol(HIP_SYMBOL(g_workCounts), zero, sizeof zero);
+}
+} // namespace cgs
+
 #if CGS_LIGHTS_TU
 namespace cgs
 {
+hipError_t workCountsLights(unsigned long long* out, bool reset) { return addWorkCounts(out, reset); }
+
 hipError_t launchRenderLights(const SceneDev& sc, const PersistArgs& pa, const void* argsDev, hipStream_t s)
 {
     Persist ps {pa.stack, pa.counter, pa.chunk};
@@ -1979,6 +1994,8 @@ hipError_t launchRenderLights(const SceneDev& sc, const PersistArgs& pa, const v
 #elif CGS_SAMPLED_TU
 namespace cgs
 {
+hipError_t workCountsSampled(unsigned long long* out, bool reset) { return addWorkCounts(out, reset); }
+
 hipError_t launchRenderSampled(const SceneDev& sc, const PersistArgs& pa, const void* argsDev, hipStream_t s)
 {
     Persist ps {pa.stack, pa.counter, pa.chunk};
@@ -2202,8 +2219,7 @@ hipError_t launchRender(const SceneDev& sc, const PersistArgs& pa, const float* 
     if (e != hipSuccess) return e;
     Persist ps {pa.stack, pa.counter, pa.chunk};
     if (samples > 0) return launchRenderSampled(sc, pa, argsDev, s);
-    // (a counting build counts in this translation unit's kernels only)
-    if (sc.nlight >= kListLights && !CGS_WORK_COUNTS) return launchRenderLights(sc, pa, argsDev, s);
+    if (sc.nlight >= kListLights) return launchRenderLights(sc, pa, argsDev, s);
     if (sc.big)
         hipLaunchKernelGGL(kRender<true>, dim3(pa.grid), dim3(256), 0, s, sc, ps, (const RenderArgs*)argsDev);
     else
@@ -2255,12 +2271,10 @@ hipError_t launchTileOrder(const uint32_t* ticks, uint32_t n, uint32_t* order, h
 // copies kWorkEvents totals to `out` and clears them when `reset`.
 hipError_t workCounts(unsigned long long* out, bool reset)
 {
-    hipError_t e = hipMemcpyFromSymbol(out, HIP_SYMBOL(g_workCounts), sizeof(g_workCounts));
-    if (e == hipSuccess && reset)
-    {
-        const unsigned long long zero[kWorkEvents] = {};
-        e = hipMemcpyToSymbol(HIP_SYMBOL(g_workCounts), zero, sizeof zero);
-    }
+    std::fill(out, out + kWorkEvents, 0ull);
+    hipError_t e = addWorkCounts(out, reset);
+    if (e == hipSuccess) e = workCountsLights(out, reset);
+    if (e == hipSuccess) e = workCountsSampled(out, reset);
     return e;
 }
 
