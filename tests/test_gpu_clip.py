@@ -44,6 +44,20 @@ def subdivide_equal(ctx, oracle, rays, P, threshold):
     assert_bits_equal(g[:, :3], o[:, :3], "t,u,v")
 
 
+@pytest.mark.parametrize("n", [40_003, 70_003, 100_003, 131_137])
+def test_pairs_of_full_waves(ctx, oracle, n):
+    """16 to 64 pairs a wave, with a remainder: waves whose lanes share only when
+    some have ended, and waves that hold more than one load of pairs."""
+    say("bezier_clip, subdivision: pairs", n)
+    rays, P = random_patch_pairs(4099, 34)
+    at = np.arange(n) % 4099
+    for method in (0, 1):
+        g = ctx.subdivision(rays[at], P[at], 0.25) if method else ctx.bezier_clip(rays[at], P[at])
+        o, _ = oracle.clip_batch(rays, P, method=method, **(dict(threshold=0.25) if method else {}))
+        assert np.array_equal(g.view(np.uint32)[:, 3] == 1, o[at, 3] == 1)
+        assert_bits_equal(g[:, :3], o[at, :3], "t,u,v")
+
+
 def grazing_pairs(n, seed):
     """Rays nearly in the plane of nearly flat patches: hundreds of passes over
     as many regions, shared by the whole wave."""
