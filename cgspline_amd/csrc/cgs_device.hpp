@@ -66,7 +66,6 @@ struct V3 { float x, y, z; };
 
 // glibc x86-64 fminf/fmaxf (the reference's host fmin/fmax): a NaN operand
 // yields the other operand, ties return the second operand.
-CGS_DEV float fmin_(float a, float b) { return (a < b || b != b) ? a : b; }
 CGS_DEV float fmax_(float a, float b) { return (a > b || b != b) ? a : b; }
 
 CGS_DEV V3 add3(V3 a, V3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
@@ -307,13 +306,12 @@ CGS_DEV bool triangleOrigin(V2& coord, V2 P, V2 A, V2 B)
 // ---------------------------------------------------------------------------
 struct ClipRay
 {
-    V3 o, d, ax0, ax1;
+    V3 o, ax0, ax1;
 };
 CGS_DEV ClipRay makeClipRay(V3 o, V3 dir)
 {
     ClipRay r;
     r.o = o;
-    r.d = dir;
     V3 e {dir.x + 0.0f, dir.y + 0.0f, dir.z + 8.0f};
     r.ax0 = versor3(cross3(dir, e));
     r.ax1 = versor3(cross3(dir, r.ax0));

@@ -342,7 +342,7 @@ CGS_DEV int dirOctant(V3 Dinv)
 
 // A shadow ray's own surface patch, clipped last.  An any-hit answer is the
 // OR of the patch tests the traversal reaches, in whatever order, so a query
-// may pass over one patch, note that the traversal reached it (`seen`), and
+// may pass over one patch, note that the traversal reached it, and
 // clip it only if no other patch is hit (sceneQuery).  A shadow ray that
 // grazes its origin patch clips it for up to thousands of passes; one that
 // another patch occludes then never does.
@@ -350,7 +350,6 @@ struct OriginSkip
 {
     int32_t object;
     uint32_t patch;
-    bool seen;
 };
 
 // ---------------------------------------------------------------------------
@@ -475,7 +474,7 @@ struct NoList
 };
 template<int METHOD, bool ANY, bool BIG, bool ORIGIN = false, class List = NoList>
 CGS_DEV bool sceneQuery(bool run, const SceneDev& sc, const NodeCache& nc, const LaneMem& lm, V3 o, V3 d, float tmax,
-                        const TraceParams& tp, ClosestHit& h, bool& overflow, OriginSkip origin = {-1, EMPTY, false},
+                        const TraceParams& tp, ClosestHit& h, bool& overflow, OriginSkip origin = {-1, EMPTY},
                         List list = List {})
 {
     constexpr bool LIST = List::kList;
@@ -770,12 +769,12 @@ CGS_DEV void addWave(unsigned long long* ctr, unsigned long long v)
     if ((threadIdx.x & 63) == 0 && v) atomicAdd(ctr, v);
 }
 
-// Persistent launches: the grid holds exactly the resident waves; each wave
-// takes chunks of 64 work items (fewer in a small launch) from a counter.  `lane` indexes the region
-// stack slice of this lane.
+// Persistent launches: the grid holds at most the resident waves; each wave takes
+// chunks of work items (64, fewer in a small launch, the caller's number in a
+// batch) from a counter.
 struct Persist
 {
-    float2* stack;
+    float2* stack;           // the waves' region stacks
     unsigned int* counter;
     uint32_t chunk;          // work items a wave takes at a time
 };
@@ -900,27 +899,23 @@ CGS_DEV uint32_t jobOf(const Job* __restrict__ jobs, uint32_t njobs, uint32_t r)
 }
 
 // Batched ray queries over many resident scenes in one launch: rays of all
-// jobs are numbered consecutively and waves take chunks of `chunk` rays (a
-// multiple of 64) from one counter, so small and large jobs share the grid
+// jobs are numbered consecutively and waves take chunks of rays (a
+// multiple of 64, ps.chunk) from one counter, so small and large jobs share the grid
 // without a launch per scene.  Each lane finds its job by binary search over
 // the jobs' first ray numbers and runs the same per-ray query as
 // kTraceClosest / kTraceAny, with the same leaf methods and polish.
 template<int METHOD, bool POLISH, bool BIG, int WAVES = CGS_BATCH_WAVES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void kTraceBatch(
-    const BatchJob* __restrict__ jobs, uint32_t njobs, uint32_t total, uint32_t chunk, Persist ps,
+    const BatchJob* __restrict__ jobs, uint32_t njobs, uint32_t total, Persist ps,
     unsigned long long* __restrict__ overflowCount, TraceParams tp)
 {
     __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     const NodeCache none {nullptr, 0};
     unsigned long long nOverflow = 0;
-    while (true)
+    for (uint32_t base = nextChunk(ps); base < total; base = nextChunk(ps))
     {
-        uint32_t base = 0;
-        if ((threadIdx.x & 63) == 0) base = atomicAdd(ps.counter, chunk);
-        base = __shfl(base, 0, 64);
-        if (base >= total) break;
-        const uint32_t end = base + chunk < total ? base + chunk : total;
+        const uint32_t end = base + ps.chunk < total ? base + ps.chunk : total;
         for (uint32_t r0 = base; r0 < end; r0 += 64)
         {
             const uint32_t r = r0 + (threadIdx.x & 63);
@@ -1598,7 +1593,7 @@ struct ShadowList
                     __uint_as_float(w[kShadowZ * 64 + at])};
         lightVector(tmax, d, P, sc.lights[l0 + (e >> 6)]);
         o = add3(P, mul3(*eps, d));
-        origin = {(int32_t)w[kShadowObject * 64 + at], w[kShadowPatch * 64 + at], false};
+        origin = {(int32_t)w[kShadowObject * 64 + at], w[kShadowPatch * 64 + at]};
         return true;
     }
     CGS_DEV void done(bool hit, bool over) const { w[kShadowFields * 64 + k] |= (hit ? kHit : 0u) | (over ? kOver : 0u); }
@@ -1703,7 +1698,7 @@ CGS_DEV V3 rayRadiance(bool run, const SceneDev& sc, const NodeCache& nc, const 
                 shadows.open(l0, n);
                 ClosestHit unused;
                 bool none = false;
-                sceneQuery<Clip, true, BIG, true>(false, sc, nc, lm, V3 {}, V3 {}, 0.0f, tp, unused, none, {-1, EMPTY, false},
+                sceneQuery<Clip, true, BIG, true>(false, sc, nc, lm, V3 {}, V3 {}, 0.0f, tp, unused, none, {-1, EMPTY},
                                                   shadows);
                 waveOrder();
                 n = 0;
@@ -1732,7 +1727,7 @@ CGS_DEV V3 rayRadiance(bool run, const SceneDev& sc, const NodeCache& nc, const 
                 if (lit) so = add3(Pt, mul3(*eps, L));
                 ClosestHit unused;
                 const bool occluded = sceneQuery<Clip, true, BIG, true>(lit, sc, nc, lm, so, L, d, tp, unused, overflow,
-                                                                        {h.object, h.patch, false});
+                                                                        {h.object, h.patch});
                 if (lit && !occluded) addLight(li, d, dotNL, L);
             }
         if (!run) continue;
@@ -1903,7 +1898,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
 // staged in LDS as in the render; otherwise each job's own scene is used.
 template<bool ONE_SCENE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_WAVES))) void kShade(
-    SceneDev sc0, const ShadeJob* __restrict__ jobs, uint32_t njobs, uint32_t total, uint32_t chunk, Persist ps,
+    SceneDev sc0, const ShadeJob* __restrict__ jobs, uint32_t njobs, uint32_t total, Persist ps,
     unsigned long long* __restrict__ counts)
 {
     __shared__ uint32_t ringLds[kRingWords], clipLds[kClipGroupWords];
@@ -1915,13 +1910,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CGS_RENDER_
     }
     const LaneMem lm = laneMem(ringLds, clipLds, ps.stack);
     uint32_t nPrimary = 0, nShadow = 0, nSecondary = 0, nOverflow = 0;
-    while (true)
+    for (uint32_t base = nextChunk(ps); base < total; base = nextChunk(ps))
     {
-        uint32_t base = 0;
-        if ((threadIdx.x & 63) == 0) base = atomicAdd(ps.counter, chunk);
-        base = __shfl(base, 0, 64);
-        if (base >= total) break;
-        const uint32_t end = base + chunk < total ? base + chunk : total;
+        const uint32_t end = base + ps.chunk < total ? base + ps.chunk : total;
         for (uint32_t r0 = base; r0 < end; r0 += 64)
         {
             const uint32_t r = r0 + (threadIdx.x & 63);
@@ -2031,11 +2022,6 @@ hipError_t persistentGrid(PersistKernel k, uint32_t& blocksPerCU)
     return e;
 }
 
-// Trace launches with an explicit leaf method.  The opt-in modes use the
-// default kernels' grid (the same VGPR budget and LDS; they spill to scratch
-// where the default kernels do not).  The default kernels clip at the fixed
-// 2^-12, so a clipping run with another tolerance takes the capped kernels
-// with a cap no run reaches (2^32 - 1 passes).
 // The least float x whose square root is at least tol, so that
 // sqrt(x) < tol is x < tolSquare(tol) (the correctly rounded square root is
 // monotone): two compares per clipping pass instead of two square roots.
@@ -2054,6 +2040,11 @@ static float tolSquare(float tol)
     return std::bit_cast<float>(hi);
 }
 
+// Trace launches with an explicit leaf method.  The opt-in modes use the
+// default kernels' grid (the same VGPR budget and LDS; they spill to scratch
+// where the default kernels do not).  The default kernels clip at the fixed
+// 2^-12, so a clipping run with another tolerance takes the capped kernels
+// with a cap no run reaches (2^32 - 1 passes).
 static TraceParams traceParams(const TraceMode& m)
 {
     return {tolSquare(m.tol), m.threshold, m.maxIters ? m.maxIters : 0xFFFFFFFFu};
@@ -2112,11 +2103,11 @@ hipError_t launchTraceBatch(const BatchJob* jobs, uint32_t njobs, uint32_t total
         if (batchAtTwoWaves(total)) grid = std::min(grid, 2u * 256u);
         const auto kernel = batchAtTwoWaves(total) ? (big ? kTraceBatch<Clip, false, true, 2> : kTraceBatch<Clip, false, false, 2>)
                                                    : (big ? kTraceBatch<Clip, false, true> : kTraceBatch<Clip, false, false>);
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, jobs, njobs, total, chunk, ps, overflow, tp);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, jobs, njobs, total, ps, overflow, tp);
         return hipGetLastError();
     }
 #define CGS_LAUNCH_BATCH(M, P) \
-    hipLaunchKernelGGL((kTraceBatch<M, P, true>), dim3(grid), dim3(256), 0, s, jobs, njobs, total, chunk, ps, overflow, tp)
+    hipLaunchKernelGGL((kTraceBatch<M, P, true>), dim3(grid), dim3(256), 0, s, jobs, njobs, total, ps, overflow, tp)
     if (m.method == CGS_METHOD_SUBDIVISION)
     {
         if (m.polish) CGS_LAUNCH_BATCH(Subdiv, true);
@@ -2176,9 +2167,9 @@ hipError_t launchShade(const SceneDev* one, const ShadeJob* jobs, uint32_t njobs
     if (total == 0 || njobs == 0) return hipSuccess;
     Persist ps {stack, counter, chunk};
     if (one)
-        hipLaunchKernelGGL(kShade<true>, dim3(grid), dim3(256), 0, s, *one, jobs, njobs, total, chunk, ps, counts);
+        hipLaunchKernelGGL(kShade<true>, dim3(grid), dim3(256), 0, s, *one, jobs, njobs, total, ps, counts);
     else
-        hipLaunchKernelGGL(kShade<false>, dim3(grid), dim3(256), 0, s, SceneDev {}, jobs, njobs, total, chunk, ps,
+        hipLaunchKernelGGL(kShade<false>, dim3(grid), dim3(256), 0, s, SceneDev {}, jobs, njobs, total, ps,
                            counts);
     return hipGetLastError();
 }

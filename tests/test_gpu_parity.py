@@ -236,7 +236,7 @@ def test_trace_past_the_sibling_ring_bitexact(ctx, oracle, grazing):
 
 def test_trace_deep_top_level_bitexact(ctx, oracle, stacked):
     """180,000 stacked objects: rays postpone 17 top-level siblings at once,
-    so past the ring's 8 the traversal reads a sibling whose heap key is 512
+    so past the ring's 8 the traversal reads a sibling whose heap key is 256
     or more (not staged in LDS) through the top level's perfect hash.  Hits
     and occlusion equal the oracle's."""
     sc, rays = stacked
