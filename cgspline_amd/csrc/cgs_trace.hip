@@ -1779,12 +1779,11 @@ CGS_DEV V3 rayRadiance(bool run, const SceneDev& sc, const NodeCache& nc, const 
 }
 
 // Occupancy target of the render megakernel (waves per SIMD): the compiler
-// keeps VGPR + AGPR use within 512 / CGS_RENDER_WAVES.  With shadow rays
-// clipping their origin patch last, two waves per SIMD (256 registers)
-// render the 1M-patch frame in 9.0 ms against 9.4 ms with three (one wave:
-// the same as two) and Test152 in 114 ms against 129 ms; the sampled render
-// is the same either way.  (Before that change, when waves waited on
-// grazing origin clips, three waves measured best.)
+// keeps VGPR + AGPR use within 512 / CGS_RENDER_WAVES.  Two (256 registers, none
+// spilled in the plain renders): at three the frame of 4,096 displaced grids
+// takes 5.4-5.6 ms against 6.1-6.3, but a 256x256 height field 324-335 us against
+// 294, a 768x768 sampled frame 8.4-10.6 ms against 7.3-9.3, and the tea frame of
+// 51 lights 112 ms against 64.
 // BIG: the scene has a BVH hashed with the wide family or a surface with a
 // cull tree (kernels for other scenes leave those paths out and keep their
 // registers).

@@ -264,7 +264,10 @@ cgs_status cgs_bezier_clip(cgs_ctx* ctx, const cgs_ray* rays, const float* patch
 
 /* spline::doSubdivision (Spline.h:495-500, Spline_Subdivision.cu:168-288),
  * batched like cgs_bezier_clip; `threshold` is the parametric size below
- * which a region is reported (reference default 2^-4). */
+ * which a region is reported (reference default 2^-4).  Regions are cut in
+ * FP32 parameters: below a threshold of 2^-23 a region may stop shrinking
+ * before it is reported, and the call may then not end in sensible time, as
+ * the reference's. */
 cgs_status cgs_subdivision(cgs_ctx* ctx, const cgs_ray* rays, const float* patches, uint32_t n,
                            float threshold, cgs_hit* hits, void* stream);
 
